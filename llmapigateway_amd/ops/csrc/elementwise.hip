@@ -193,7 +193,11 @@ __global__ void rmsnorm_wave_kernel(
 // many: 300 rows of 4096 with the addition 4.5 us (a wave a row 6.2, 256 threads
 // in pieces 4.9), 256 rows of 3584 3.7 (8.8, 4.4), 4096 rows of 4096 23.8 (25.9
 // in pieces), 5.6 TB/s.
-template <bool FUSED_RESIDUAL, int THREADS>
+//
+// The sum of squares is that of 64 or 256 threads (LIKE) which take the row's
+// pieces in turn, to the last bit, so that a row's norm does not depend on which
+// of the kernels here has it: pieces meet in LDS where there are more threads.
+template <bool FUSED_RESIDUAL, int THREADS, int LIKE>
 __launch_bounds__(THREADS)
 __global__ void rmsnorm_row_kernel(
     bf16* __restrict__ out, const bf16* __restrict__ x,
@@ -201,47 +205,59 @@ __global__ void rmsnorm_row_kernel(
     const int64_t row = (int64_t)blockIdx.x * H;
     const int at = threadIdx.x * 8;
     const bool in = at < H;
-    uint4 g = {0, 0, 0, 0};
+    uint4 v = {0, 0, 0, 0}, g = {0, 0, 0, 0};
     float f[8] = {};
+    auto unpack = [](const uint4& u, float* to) {
+        unpack2(u.x, to[0], to[1]);
+        unpack2(u.y, to[2], to[3]);
+        unpack2(u.z, to[4], to[5]);
+        unpack2(u.w, to[6], to[7]);
+    };
     if (in) {
-        const uint4 vx = *reinterpret_cast<const uint4*>(x + row + at);
+        v = *reinterpret_cast<const uint4*>(x + row + at);
         g = *reinterpret_cast<const uint4*>(weight + at);
-        unpack2(vx.x, f[0], f[1]);
-        unpack2(vx.y, f[2], f[3]);
-        unpack2(vx.z, f[4], f[5]);
-        unpack2(vx.w, f[6], f[7]);
+        unpack(v, f);
         if (FUSED_RESIDUAL) {
             const uint4 vr = *reinterpret_cast<const uint4*>(residual + row + at);
             float r[8];
-            unpack2(vr.x, r[0], r[1]);
-            unpack2(vr.y, r[2], r[3]);
-            unpack2(vr.z, r[4], r[5]);
-            unpack2(vr.w, r[6], r[7]);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) f[j] = bfbits2f(f2bfbits(f[j] + r[j]));
-            *reinterpret_cast<uint4*>(residual + row + at) = make_uint4(
-                pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]), pack2(f[6], f[7]));
+            unpack(vr, r);
+            v = make_uint4(pack2(f[0] + r[0], f[1] + r[1]), pack2(f[2] + r[2], f[3] + r[3]),
+                           pack2(f[4] + r[4], f[5] + r[5]), pack2(f[6] + r[6], f[7] + r[7]));
+            *reinterpret_cast<uint4*>(residual + row + at) = v;
+            unpack(v, f);
         }
     }
     float ssq = 0.f;
+    if constexpr (THREADS > LIKE) {
+        __shared__ uint4 pieces[THREADS];
+        pieces[threadIdx.x] = v;
+        __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 8; ++j) ssq += f[j] * f[j];
+        for (int t = 0; t < THREADS / LIKE; ++t) {
+            float p[8];
+            unpack(pieces[threadIdx.x % LIKE + t * LIKE], p);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) ssq = fmaf(p[j], p[j], ssq);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ssq = fmaf(f[j], f[j], ssq);
+    }
     ssq = wave_reduce_sum(ssq);
-    if (THREADS > WAVE_SIZE) {
-        __shared__ float red[THREADS / WAVE_SIZE];
-        if ((threadIdx.x & (WAVE_SIZE - 1)) == 0) red[threadIdx.x / WAVE_SIZE] = ssq;
+    constexpr int WAVES = (THREADS < LIKE ? THREADS : LIKE) / WAVE_SIZE;
+    if (WAVES > 1) {
+        __shared__ float red[WAVES];
+        if ((threadIdx.x & (WAVE_SIZE - 1)) == 0 && threadIdx.x < WAVES * WAVE_SIZE)
+            red[threadIdx.x / WAVE_SIZE] = ssq;
         __syncthreads();
         ssq = 0.f;
 #pragma unroll
-        for (int w = 0; w < THREADS / WAVE_SIZE; ++w) ssq += red[w];
+        for (int w = 0; w < WAVES; ++w) ssq += red[w];
     }
     const float inv = rsqrtf(ssq / (float)H + eps);
     if (!in) return;
     float w8[8];
-    unpack2(g.x, w8[0], w8[1]);
-    unpack2(g.y, w8[2], w8[3]);
-    unpack2(g.z, w8[4], w8[5]);
-    unpack2(g.w, w8[6], w8[7]);
+    unpack(g, w8);
     *reinterpret_cast<uint4*>(out + row + at) = make_uint4(
         pack2(f[0] * inv * w8[0], f[1] * inv * w8[1]),
         pack2(f[2] * inv * w8[2], f[3] * inv * w8[3]),
@@ -249,13 +265,22 @@ __global__ void rmsnorm_row_kernel(
         pack2(f[6] * inv * w8[6], f[7] * inv * w8[7]));
 }
 
+// up to 1024 rows of up to 8 times 512 columns are summed as by a wave a row,
+// others as by 256 threads
 template <bool FUSED>
 static hipError_t launch_rms_row(bf16* out, const bf16* x, bf16* residual,
                                  const bf16* w, float eps, int T, int H,
                                  hipStream_t stream) {
+    const bool wave = T <= 1024 && H <= 4096 && H % 512 == 0;
 #define RMS_R(THREADS)                                                         \
-    rmsnorm_row_kernel<FUSED, THREADS>                                         \
-        <<<T, THREADS, 0, stream>>>(out, x, residual, w, eps, H)
+    do {                                                                       \
+        if (wave)                                                              \
+            rmsnorm_row_kernel<FUSED, THREADS, 64>                             \
+                <<<T, THREADS, 0, stream>>>(out, x, residual, w, eps, H);      \
+        else                                                                   \
+            rmsnorm_row_kernel<FUSED, THREADS, 256>                            \
+                <<<T, THREADS, 0, stream>>>(out, x, residual, w, eps, H);      \
+    } while (0)
     if (H <= 512) RMS_R(64);
     else if (H <= 1024) RMS_R(128);
     else if (H <= 2048) RMS_R(256);
