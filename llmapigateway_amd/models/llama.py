@@ -139,23 +139,23 @@ class LlamaModel:
         return x
 
     def _row_parallel(self, x: torch.Tensor, w: torch.Tensor,
-                      w_swz=None) -> torch.Tensor:
+                      w_swz=None, linear=ops.linear) -> torch.Tensor:
         """Row-parallel linear with comm/compute overlap: split the token
         batch in two, launch the first half's all-reduce asynchronously
         while the second half's GEMM runs (overlap the 2
         all-reduces/layer with compute). Falls back to the plain form for
         tiny batches or TP=1."""
         if self.tp_group is None:
-            return ops.linear(x, w, w_swz)
+            return linear(x, w, w_swz)
         T = x.shape[0]
         if T < 32:  # split overhead exceeds the overlap win
-            y = ops.linear(x, w, w_swz)
+            y = linear(x, w, w_swz)
             dist.all_reduce(y, group=self.tp_group)
             return y
         half = T // 2
-        y1 = ops.linear(x[:half], w, w_swz)
+        y1 = linear(x[:half], w, w_swz)
         h1 = dist.all_reduce(y1, group=self.tp_group, async_op=True)
-        y2 = ops.linear(x[half:], w, w_swz)
+        y2 = linear(x[half:], w, w_swz)
         h2 = dist.all_reduce(y2, group=self.tp_group, async_op=True)
         h1.wait()
         h2.wait()
@@ -184,12 +184,21 @@ class LlamaModel:
         ksc = k_scales if k_scales is not None else [None] * len(self.layers)
         vsc = v_scales if v_scales is not None else [None] * len(self.layers)
         T = batch.token_ids.shape[0]
-        if self.tp_group is None and self.layers:
-            first = self.layers[0]  # all are alike
+        first = self.layers[0] if self.layers else {}  # all are alike
+        # A prompt's rows that become bytes are summed in the order they have always
+        # been. Where larger steps have separate kernels, a prompt that starts from
+        # pages has them too: it is rounded at the same places as if it were whole.
+        in_order = bool(first) and batch.kind != "decode" and (
+            k_scales is not None
+            or batch.cached_lens is not None and not ops.layer_tiles(256, first, c.head_dim)
+        )
+        if self.tp_group is None and first and not in_order:
             if ops.layer_streams(T, first):
                 return self._forward_streamed(batch, k_caches, v_caches, ksc, vsc)
             if ops.layer_tiles(T, first, c.head_dim):
                 return self._forward_tiled(batch, k_caches, v_caches, ksc, vsc)
+        linear = ops.linear_in_order if in_order else ops.linear
+        swiglu_linear = ops.swiglu_linear_in_order if in_order else ops.swiglu_linear
         h = F.embedding(batch.token_ids, self.embed)
         residual = h  # placeholder; layer 0 sets the real residual stream
 
@@ -199,7 +208,7 @@ class LlamaModel:
             else:
                 x, residual = ops.rmsnorm_residual(h, residual, layer["input_norm"], c.rms_eps)
 
-            qkv = ops.linear(x, layer["qkv"], layer.get("qkv_swz"))
+            qkv = linear(x, layer["qkv"], layer.get("qkv_swz"))
             q, k, v = self._heads(qkv)
             ops.rope_and_kv_write(
                 q, k, v, k_caches[i], v_caches[i],
@@ -208,21 +217,23 @@ class LlamaModel:
             )
             attn = self._attend(batch, q, k, v, k_caches[i], v_caches[i], ksc[i], vsc[i])
             h = self._row_parallel(
-                attn.reshape(T, c.q_size), layer["o"], layer.get("o_swz")
+                attn.reshape(T, c.q_size), layer["o"], layer.get("o_swz"), linear
             )
 
             x, residual = ops.rmsnorm_residual(h, residual, layer["post_norm"], c.rms_eps)
             h = self._row_parallel(
-                ops.swiglu_linear(
+                swiglu_linear(
                     x, layer["gate_up"], layer.get("gate_up_swz"),
                     layer.get("gate_up_int"),
                 ),
-                layer["down"], layer.get("down_swz"),
+                layer["down"], layer.get("down_swz"), linear,
             )
 
         x, _ = ops.rmsnorm_residual(h, residual, self.final_norm, c.rms_eps)
         if batch.logits_indices is not None:
             x = x[batch.logits_indices]
+        if in_order:
+            return ops.linear_in_order(x, self.lm_head, head=True).float()
         return ops.linear(x, self.lm_head).float()
 
     def _forward_streamed(

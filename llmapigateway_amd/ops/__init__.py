@@ -519,6 +519,13 @@ def linear(
         y = torch.empty((M, w.shape[0]), dtype=torch.bfloat16, device=x.device)
         _shared().gemm_stream(y, x, w, False)
         return y
+    return _linear_slabs(x, w, w_swz)
+
+
+def _linear_slabs(
+    x: torch.Tensor, w: torch.Tensor, w_swz: Optional[torch.Tensor] = None
+) -> torch.Tensor:
+    M = x.shape[0]
     if (
         x.is_cuda
         and x.dtype == torch.bfloat16
@@ -556,6 +563,52 @@ def linear(
             _shared().gemm_skinny(y, x, w, ws, nsk, False)
             return y
     return torch.nn.functional.linear(x, w)
+
+
+# ---- a prompt's products in an order that does not change ----
+# What a prompt leaves in pages of e4m3 is bytes: a sum in another order turns
+# none of bf16's digits that count, but moves a quarter of the codes after four
+# layers. So the rows of a prompt have their sums where they have always been:
+# up to 16 by gemm_skinny, up to 256 as gemm_m256 sums (from the weight as it
+# lies: gemm_tile in the same splits of K), others by the library.
+
+
+def linear_in_order(
+    x: torch.Tensor, w: torch.Tensor, w_swz: Optional[torch.Tensor] = None,
+    head: bool = False,
+) -> torch.Tensor:
+    """linear() of one of a layer's weights, in the order that a fragment-major
+    twin gives, whether there is one or not; heads have none."""
+    if w_swz is None and not head and x.is_cuda and 8 < x.shape[0] <= 256 and _twin_fits(w):
+        (M, K), N = x.shape, w.shape[0]
+        cfg = _m256_config(M, N, K)
+        if cfg is not None and _streamable(x, w):
+            parts = torch.empty((cfg["nsk"], M, N), dtype=torch.float32, device=x.device)
+            _native().gemm_tile(parts, x, w, True)
+            y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+            _native().sum_parts(y, parts)
+            return y
+    return _linear_slabs(x, w, w_swz)
+
+
+def _twin_fits(w: torch.Tensor) -> bool:
+    return _tileable(w) and w.shape[0] % 64 == 0 and not os.environ.get("LLMAPI_NO_FRAG_WEIGHTS")
+
+
+def swiglu_linear_in_order(
+    x: torch.Tensor, w: torch.Tensor,
+    w_swz: Optional[torch.Tensor] = None,
+    w_int: Optional[torch.Tensor] = None,
+) -> torch.Tensor:
+    """swiglu_linear() in the same way."""
+    cfg = _m256_swiglu_config(x.shape[0], *w.shape) if x.is_cuda else None
+    if cfg is not None and w_int is not None:
+        return gemm_m256_swiglu(x, w_int, **cfg)
+    if cfg is not None and _twin_fits(w) and _streamable(x, w):
+        y = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype, device=x.device)
+        _native().gemm_tile(y, x, w, True)
+        return y
+    return swiglu(linear_in_order(x, w, w_swz))
 
 
 # ---- a decode step's products with what stands beside them ----

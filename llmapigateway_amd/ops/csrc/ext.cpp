@@ -18,7 +18,8 @@ hipError_t launch_sample(int64_t*, const float*, const float*, const float*, flo
 hipError_t launch_topk_topp_filter(float*, const float*, const int*, int, int, void*, hipStream_t);
 size_t filter_scratch_bytes(int, int);
 hipError_t launch_gemm_stream_qkv(void*, const void*, const void*, int, int, const void*, float, const int64_t*, const float*, const int64_t*, void*, void*, int, int, int, int, hipStream_t);
-hipError_t launch_gemm_tile(void*, const void*, const void*, int, int, int, int, int, hipStream_t);
+hipError_t launch_gemm_tile(void*, const void*, const void*, int, int, int, int, int, int, hipStream_t);
+hipError_t launch_gemm_reduce(void*, const float*, int64_t, int, hipStream_t);
 int gemm_tile_splits(int, int, int);
 hipError_t launch_add_parts_norm(void*, void*, const float*, const void*, float, int, int, int, hipStream_t);
 hipError_t launch_embed_norm(void*, void*, const int64_t*, const void*, const void*, float, int, int64_t, int, hipStream_t);
@@ -329,8 +330,8 @@ void gemm_stream_rows(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t
 }
 
 // y = x @ w.T in fp32 (y [M, N]) or as parts to be added up (y [splits, M, N]),
-// or silu(gate) * up of it (y bf16 [M, N / 2])
-void gemm_tile(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
+// or silu(gate) * up of it (y bf16 [M, N / 2]); in_order: sums by rising depth
+void gemm_tile(torch::Tensor y, torch::Tensor x, torch::Tensor w, bool in_order) {
     check_bf16(x, "x");
     check_bf16(w, "w");
     TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && dense16(x) && dense16(w));
@@ -342,7 +343,18 @@ void gemm_tile(torch::Tensor y, torch::Tensor x, torch::Tensor w) {
     TORCH_CHECK(swiglu || y.scalar_type() == torch::kFloat32);
     CHECK_HIP(launch_gemm_tile(y.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K,
                                parts ? (int)y.size(0) : 1, swiglu ? 1 : parts ? 2 : 0,
-                               current_stream()));
+                               in_order ? 1 : 0, current_stream()));
+}
+
+// y = the sum of parts [splits, M, N], one after the other
+void sum_parts(torch::Tensor y, torch::Tensor parts) {
+    check_bf16(y, "y");
+    TORCH_CHECK(parts.is_cuda() && parts.scalar_type() == torch::kFloat32 && parts.dim() == 3);
+    TORCH_CHECK(dense16(y) && dense16(parts) && y.dim() == 2 && y.numel() > 0);
+    TORCH_CHECK(parts.size(0) > 0 && parts.size(1) == y.size(0) && parts.size(2) == y.size(1) &&
+                y.size(1) % 4 == 0);
+    CHECK_HIP(launch_gemm_reduce(y.data_ptr(), parts.data_ptr<float>(), y.numel(),
+                                 (int)parts.size(0), current_stream()));
 }
 
 // r += sum of parts; out = rmsnorm(r)
@@ -473,7 +485,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "macro-tile LDS-staged decode GEMM y = x @ w.T (M <= 256)");
     m.def("gemm_stream_rows", &gemm_stream_rows,
           "products of few rows with the norm in front, swiglu or the addition behind");
-    m.def("gemm_tile", &gemm_tile, "x @ w.T of up to 256 rows: fp32, in parts, or swiglu");
+    m.def("gemm_tile", &gemm_tile,
+          "x @ w.T of up to 256 rows (in parts 512): fp32, in parts, or swiglu",
+          py::arg("y"), py::arg("x"), py::arg("w"), py::arg("in_order") = false);
+    m.def("sum_parts", &sum_parts, "sum of parts in bf16");
     m.def("gemm_tile_splits", &gemm_tile_splits, "how many parts suit a product");
     m.def("add_parts_norm", &add_parts_norm, "sum of parts onto the stream, and its norm");
     m.def("embed_norm", &embed_norm, "rows of the embedding, and their norm");

@@ -8,7 +8,8 @@
 // (parts_rows.hip): a sum of its own took 4.3 to 5.5 us. Workgroups of one column
 // tile start at different depths, so that rows of W at one stride do not all ask
 // the same memory channels at once (28672 x 4096: 53 us without, 47.8 with; 128256
-// x 4096: 233 and 199). Above, transfers and products bound it together: 65536 x
+// x 4096: 233 and 199); not where the order of sums is asked for, which is that of
+// depth then. Above, transfers and products bound it together: 65536 x
 // 4096 at 256 rows takes 136 us, its transfers alone 98, its products alone 99.
 //
 // us, with what reads the parts, against what ran before (the library, tiles over
@@ -55,7 +56,7 @@ template <int BM, int BN, int WM, int WN, int NX, int NW, TileLeaves OUT>
 __launch_bounds__(WM* WN* WAVE_SIZE, 2)
 __global__ void gemm_tile_kernel(
     void* __restrict__ y, const bf16* __restrict__ x, const bf16* __restrict__ w,
-    int M, int N, int K, int n_tiles, int m_tiles, int splits, bool once) {
+    int M, int N, int K, int n_tiles, int m_tiles, int splits, bool once, bool in_order) {
     constexpr int ROW = 128, F = WM * WN / 2;         // bytes of a tile's row
     constexpr int XB = BM * ROW, WB = BN * ROW;
     constexpr int XMINE = BM / 8 / F, WMINE = BN / 8 / F;  // transfers of 1 KB: 8 rows
@@ -81,7 +82,7 @@ __global__ void gemm_tile_kernel(
     const int k_tiles = K / 64;
     const int each = (k_tiles + splits - 1) / splits;
     const int first = split * each, count = max(0, min(k_tiles - first, each));
-    const int turn = splits == 1 && count > 0 ? (n_tile * 5) % count : 0;
+    const int turn = splits == 1 && count > 0 && !in_order ? (n_tile * 5) % count : 0;
 
     // this wave's transfers: 8 rows of X or W each; a lane's piece lies so that
     // 16 rows at one piece cover all banks
@@ -249,10 +250,11 @@ extern "C" int gemm_tile_splits(int M, int N, int K) {
     return s < 1 ? 1 : s > 8 ? 8 : s;
 }
 
-// leaves: TileLeaves; splits: 1, or with TILE_PART what y has room for
+// leaves: TileLeaves; splits: 1, or with TILE_PART what y has room for; in_order:
+// each split's sum by rising depth
 extern "C" hipError_t launch_gemm_tile(
     void* y, const void* x, const void* w, int M, int N, int K, int splits, int leaves,
-    hipStream_t stream) {
+    int in_order, hipStream_t stream) {
     if (M <= 0 || M > (leaves == TILE_PART ? 512 : 256) || N <= 0 || N % 16 != 0 || K <= 0 || K % 64 != 0)
         return hipErrorInvalidValue;
     if ((int64_t)N * K >= (int64_t)1 << 31) return hipErrorInvalidValue;  // 32-bit offsets
@@ -266,7 +268,7 @@ extern "C" hipError_t launch_gemm_tile(
         gemm_tile_kernel<BM, BN, WM, WN, NX, NW, OUT>                          \
             <<<grid, dim3(WM * WN * WAVE_SIZE), 0, stream>>>(                  \
                 y, (const bf16*)x, (const bf16*)w, M, N, K, n_tiles, m_tiles,  \
-                splits, once);                                                 \
+                splits, once, in_order != 0);                                                 \
     } while (0)
 #define LAUNCH_O(BM, BN, WM, WN, NX, NW)                                       \
     do {                                                                       \

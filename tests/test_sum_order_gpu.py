@@ -42,3 +42,42 @@ def test_rmsnorm_order(T, H, plain, added):
     w = _rows(rs, H)
     assert _crc(ops.rmsnorm(x, w, 1e-5)) == plain
     assert _crc(ops.rmsnorm_residual(x, r, w, 1e-5)[0]) == added
+
+
+# every split of K that the fragment-major kernel has, row tiles of 64 to 256
+@pytest.mark.parametrize("M", [9, 16, 40, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize(
+    "N,K", [(4096, 4096), (4096, 8256), (3584, 3584), (2048, 1024), (8192, 8192), (8192, 8256),
+            (7168, 2048), (64, 2048)])
+def test_linear_in_order(M, N, K):
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K, device=DEV).bfloat16()
+    w = (torch.randn(N, K, device=DEV) * K**-0.5).bfloat16()
+    cfg = ops._m256_config(M, N, K)
+    got = ops.linear_in_order(x, w)
+    if cfg is None:
+        want = ops._linear_slabs(x, w)
+    else:
+        want = ops.gemm_m256(x, ops.swizzle_weight_frag(w), **cfg)
+        assert torch.equal(ops.linear_in_order(x, w, ops.swizzle_weight_frag(w)), want)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M", [9, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize("N", [28672, 7168])
+def test_swiglu_linear_in_order(M, N, K=4096):
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device=DEV).bfloat16()
+    w = (torch.randn(N, K, device=DEV) * K**-0.5).bfloat16()
+    twin = ops.swizzle_weight_frag(ops.interleave_gate_up(w))
+    want = ops.gemm_m256_swiglu(x, twin, **ops._m256_swiglu_config(M, N, K))
+    assert torch.equal(ops.swiglu_linear_in_order(x, w), want)
+    assert torch.equal(ops.swiglu_linear_in_order(x, w, w_int=twin), want)
+
+
+def test_sum_parts_refuses():
+    parts = torch.zeros(2, 4, 64, device=DEV)
+    y = torch.zeros(4, 64, device=DEV).bfloat16()
+    for args in ((y[:3], parts), (y, parts.double()), (y, parts[0]), (y[:, :32], parts)):
+        with pytest.raises(RuntimeError):
+            ops._native().sum_parts(*args)
