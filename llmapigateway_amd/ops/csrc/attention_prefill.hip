@@ -15,20 +15,25 @@
 // - Tiles are transferred to LDS without registers into one of two buffers
 //   while the other is in use, one barrier a tile. Pages of bytes pass through
 //   registers, where they become bf16 (value times scale, rounded once).
-// - The running maximum moves only when a score exceeds it by 2^8: weights stay
-//   below 2^8 (rounding is relative), and the sums are rarely rescaled.
+// - Sums are in a fixed order, which no choice of workgroups touches: 64 keys at
+//   a time, scores relative to the largest so far, weights as bf16 (the largest is
+//   1 and loses nothing) for the values and as fp32 for their sum. What a prompt
+//   leaves behind in pages of bytes so depends on the prompt alone. (A maximum
+//   that moves only past 2^8 takes 163 us instead of 185 for 4096 tokens, but
+//   rounds the largest weights, too: over 4000 keys the weights' share of the error
+//   is 1.6e-3 then, 1.25e-3 so.)
 // - Blocks of one kv head follow each other at the distance of the XCDs, and
 //   late tiles, which see the most keys, start first.
 //
 // One layer, 32 query and 8 kv heads; before: 64 rows and one head a workgroup,
 // keys and values through registers, weights through LDS:
-//   4096 tokens                   1123 us -> 157 us (875 TFLOP/s)
-//   4000 tokens after 4032        2386    -> 440    (890), e4m3 pages the same
-//   9 x 117-213 tokens after 1984  420    ->  90
-//   32 x 66-128 tokens              50    ->  23
-//   37 tokens                      6.5    -> 5.1
+//   4096 tokens                   1117 us -> 185 us (743 TFLOP/s)
+//   4000 tokens after 4032        2371    -> 503    (786), e4m3 pages the same
+//   9 x 117-213 tokens after 1984  428    -> 102
+//   32 x 66-128 tokens              46    ->  24
+//   37 tokens                      6.6    -> 6.3
 // Long prompts are bound by the vector ALU beside the matrix cores (an
-// exponential and 3.5 operations a score take as long as its products).
+// exponential and 6 operations a score, the sums' rescaling).
 
 #include "common.h"
 #include "lds_dma.h"
@@ -36,15 +41,19 @@
 
 #define PF_D 128
 #define QTILE 64  // query rows of a tile (ops.build_prefill_tiles)
+#define PF_KEYS 64  // keys of a tile
 #define PF_ROW (2 * PF_D)  // bytes
 
 namespace {
 
 // where the 16-byte piece p of a row lies, without bank conflicts: keys are
-// read 16 rows at one piece, values 4 rows a lane group at two
-__device__ __forceinline__ int pf_key_piece(int row, int p) { return p ^ (row & 15); }
+// read rows 8g + r (+ 4) of g, r < 4 at one piece, values rows 8g + r of two
+// lane groups g at two
+__device__ __forceinline__ int pf_key_piece(int row, int p) {
+    return p ^ ((row & 3) | (row >> 3 & 3) << 2);
+}
 __device__ __forceinline__ int pf_value_piece(int row, int p) {
-    return (((p >> 1) ^ (row & 7)) << 1) | (p & 1);
+    return (((p >> 1) ^ ((row & 3) | (row >> 3 & 1) << 2)) << 1) | (p & 1);
 }
 
 __device__ __forceinline__ float pf_column_max(float v) {
@@ -55,13 +64,37 @@ __device__ __forceinline__ float pf_column_max(float v) {
         __float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
-__device__ __forceinline__ float pf_column_sum(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(
-        __float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto b = __builtin_amdgcn_permlane32_swap(
-        __float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+// The sum of 64 weights of one column, of which a lane has those of keys
+// 32c + 8*grp + 4h + r at [c][4h + r]: first the four of the keys that are equal
+// in their last 4 bits, in order, then these by halves (8 apart, 4, 2, 1). A swap
+// leaves one half's two operands in each half of the lanes.
+__device__ __forceinline__ float add_in_halves(uint32_t a, uint32_t b) {
+    return __uint_as_float(a) + __uint_as_float(b);
+}
+__device__ __forceinline__ float pf_key_sum(const float (&e)[2][8]) {
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const auto a = __builtin_amdgcn_permlane32_swap(
+            __float_as_uint(e[0][r]), __float_as_uint(e[0][4 + r]), false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(
+            __float_as_uint(e[1][r]), __float_as_uint(e[1][4 + r]), false, false);
+        v[r] = add_in_halves(a[0], a[1]) + __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    }
+    float w[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const auto a = __builtin_amdgcn_permlane16_swap(
+            __float_as_uint(v[r]), __float_as_uint(v[r + 2]), false, false);
+        w[r] = add_in_halves(a[0], a[1]);
+    }
+    auto c = __builtin_amdgcn_permlane32_swap(
+        __float_as_uint(w[0]), __float_as_uint(w[1]), false, false);
+    uint32_t x = __float_as_uint(add_in_halves(c[0], c[1]));
+    c = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = __float_as_uint(add_in_halves(c[0], c[1]));
+    c = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return add_in_halves(c[0], c[1]);
 }
 
 // 16 e4m3 bytes times their row's scale as 16 bf16
@@ -79,10 +112,9 @@ __device__ __forceinline__ void dequantize16(const uint4& b, float scale, uint4*
 
 }  // namespace
 
-// HG: heads of a workgroup (two waves each); KT: keys of a tile; FP8C: pages
-// are e4m3 with a scale a row; FINE: weights enter as the sum of two bf16, as
-// in decoding, where they cost nothing that shows.
-template <int HG, int KT, bool FP8C, bool FINE>
+// HG: heads of a workgroup (two waves each); FP8C: pages are e4m3 with a scale
+// a row.
+template <int HG, bool FP8C>
 __launch_bounds__(HG * 2 * WAVE_SIZE, 2)
 __global__ void attention_prefill_kernel(
     bf16* __restrict__ out,             // [T, Hq, D]
@@ -92,8 +124,7 @@ __global__ void attention_prefill_kernel(
     const int* __restrict__ cu_seqlens, // [B+1]
     const int* __restrict__ tile_seq,   // [ntiles] sequence of each tile
     const int* __restrict__ tile_off,   // [ntiles] its first row in the sequence
-    float scale_log2,                   // |scale| * log2(e), not 0
-    uint32_t q_sign,                    // 0x80008000 where scale is negative
+    float scale,
     int G, int Hkv, int head_groups, int64_t q_stride, int64_t k_stride, int64_t v_stride,
     const char* __restrict__ k_cache,   // [NB, Hkv, BS, D] or null
     const char* __restrict__ v_cache,
@@ -102,7 +133,7 @@ __global__ void attention_prefill_kernel(
     const int* __restrict__ block_tables,  // [B, max_blocks] or null
     const int* __restrict__ cached_lens,   // [B] or null
     int block_size, int max_blocks) {
-    constexpr int NW = 2 * HG, SUBS = KT / 16, CHUNKS = KT / 32, NQ = 2;
+    constexpr int KT = PF_KEYS, NW = 2 * HG, NQ = 2;
     constexpr int TILE = KT * PF_ROW;          // bytes of a key or value tile
     constexpr int MOVES = KT / 4;              // 1 KB transfers of one
     constexpr int MINE = (MOVES + NW - 1) / NW;
@@ -131,11 +162,7 @@ __global__ void attention_prefill_kernel(
         const int r = min(row0 + n * 16 + col, seq_len - 1);
         const bf16* p = q + (int64_t)(seq_start + r) * q_stride + (int64_t)head * PF_D + grp * 8;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            uint4 raw = *reinterpret_cast<const uint4*>(p + c * 32);
-            raw.x ^= q_sign; raw.y ^= q_sign; raw.z ^= q_sign; raw.w ^= q_sign;
-            qf[n][c] = as_frag(raw);
-        }
+        for (int c = 0; c < 4; ++c) qf[n][c] = *reinterpret_cast<const bf16x8*>(p + c * 32);
     }
 
     const int limit = min(seq_len, tile0 + QTILE);  // keys that the tile sees
@@ -235,13 +262,15 @@ __global__ void attention_prefill_kernel(
 #pragma unroll
         for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(qf[n][c]));
 
-    // fragment addresses: keys u*16 + col, piece 4c + grp; values of rows
-    // 32*chunk (+ 16) + 4*grp + col/4, columns 16d + (col%4)*4
+    // fragment addresses: row i of a product's first operand is key 8(i/4) + i%4
+    // of 32 (+ 4 in the second), piece 4c + grp, so that a lane's scores are those
+    // of keys 8*grp..8*grp+7; values of these rows, columns 16d + (col%4)*4
+    const int k_row = (col >> 2) * 8 + (col & 3);
     int key_at[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-        key_at[c] = col * PF_ROW + pf_key_piece(col, c * 4 + grp) * 16;
-    const int v_row = grp * 4 + (col >> 2);
+        key_at[c] = k_row * PF_ROW + pf_key_piece(k_row, c * 4 + grp) * 16;
+    const int v_row = grp * 8 + (col >> 2);
     const int value_at = v_row * PF_ROW + ((col >> 1) & 1) * 16 + (col & 1) * 8;
 
     for (int t = 0; t < n_tiles; ++t) {
@@ -253,23 +282,39 @@ __global__ void attention_prefill_kernel(
         }
         const bool fresh = t >= n_cached;
         const int key0 = (fresh ? t - n_cached : t) * KT;
+        // behind the last key lies its row again: 0 times an infinity is none of
+        // the values' sum
+        const int rows = (fresh ? limit : cached) - key0;
+        if (rows < KT) {
+            for (int i = rows * (PF_ROW / 16) + threadIdx.x; i < TILE / 16; i += NW * WAVE_SIZE)
+                reinterpret_cast<uint4*>(lds[t & 1][1])[i] = make_uint4(0, 0, 0, 0);
+            lds_barrier();
+        }
         // rows of this wave behind all keys of the tile: nothing to do
         if (!has_head || (fresh && key0 > row0 + 31) || row0 >= seq_len) continue;
         const char* keys = lds[t & 1][0];
         const char* vals = lds[t & 1][1];
 
-        f32x4 s[NQ][SUBS];
+        float s[NQ][2][8];  // scores of keys 32c + 8*grp + j
 #pragma unroll
-        for (int u = 0; u < SUBS; ++u) {
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int n = 0; n < NQ; ++n) s[n][u] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int h = 0; h < 2; ++h) {
+                f32x4 p[NQ];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const bf16x8 kf = *reinterpret_cast<const bf16x8*>(keys + key_at[c] + u * 16 * PF_ROW);
+                for (int n = 0; n < NQ; ++n) p[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int n = 0; n < NQ; ++n) s[n][u] = mfma16(kf, qf[n][c], s[n][u]);
+                for (int d = 0; d < 4; ++d) {
+                    const bf16x8 kf =
+                        *reinterpret_cast<const bf16x8*>(keys + key_at[d] + (c * 32 + h * 4) * PF_ROW);
+#pragma unroll
+                    for (int n = 0; n < NQ; ++n) p[n] = mfma16(kf, qf[n][d], p[n]);
+                }
+#pragma unroll
+                for (int n = 0; n < NQ; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[n][c][h * 4 + r] = p[n][r] * scale;
             }
-        }
 
         // keys that some row of this wave does not see
         const int seen = fresh ? row0 + 1 : cached;
@@ -278,74 +323,61 @@ __global__ void attention_prefill_kernel(
             for (int n = 0; n < NQ; ++n) {
                 const int most = fresh ? row0 + n * 16 + col : cached - 1;
 #pragma unroll
-                for (int u = 0; u < SUBS; ++u)
+                for (int c = 0; c < 2; ++c)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (key0 + u * 16 + grp * 4 + r > most) s[n][u][r] = -INFINITY;
+                    for (int j = 0; j < 8; ++j)
+                        if (key0 + c * 32 + grp * 8 + j > most) s[n][c][j] = -INFINITY;
             }
         }
 
-        bf16x8 p[NQ][CHUNKS], p_low[NQ][FINE ? CHUNKS : 1];
         float top[NQ];
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
             float x = s[n][0][0];
 #pragma unroll
-            for (int u = 0; u < SUBS; ++u)
+            for (int c = 0; c < 2; ++c)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) x = fmaxf(x, s[n][u][r]);
-            top[n] = pf_column_max(x) * scale_log2;
+                for (int j = 0; j < 8; ++j) x = fmaxf(x, s[n][c][j]);
+            top[n] = pf_column_max(x);
         }
-        if (__any(top[0] > m[0] + 8.f || top[1] > m[1] + 8.f)) {
+        float factor[NQ] = {1.f, 1.f};
+        if (__any(top[0] > m[0] || top[1] > m[1])) {
 #pragma unroll
             for (int n = 0; n < NQ; ++n) {
                 const float m_new = fmaxf(m[n], top[n]);
-                const float factor =
-                    __builtin_amdgcn_exp2f(m[n] - (m_new == -INFINITY ? 0.f : m_new));
+                factor[n] = __expf(m[n] - (m_new == -INFINITY ? 0.f : m_new));
                 m[n] = m_new;
-                l[n] *= factor;
 #pragma unroll
                 for (int d = 0; d < 8; ++d)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[n][d][r] *= factor;
+                    for (int r = 0; r < 4; ++r) acc[n][d][r] *= factor[n];
             }
         }
+        bf16x8 p[NQ][2];
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
             const float base = m[n] == -INFINITY ? 0.f : m[n];
-            float sum = 0.f;
 #pragma unroll
-            for (int c = 0; c < CHUNKS; ++c) {
-                float e[8];
+            for (int c = 0; c < 2; ++c) {
+                float* e = s[n][c];
 #pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    e[r] = __builtin_amdgcn_exp2f(
-                        fmaf(s[n][2 * c + r / 4][r % 4], scale_log2, -base));
-                    sum += e[r];
-                }
-                if constexpr (FINE) {
-                    split_frag(e, p[n][c], p_low[n][c]);
-                } else {
-                    p[n][c] = as_frag(make_uint4(
-                        cvt_pk_bf16(e[0], e[1]), cvt_pk_bf16(e[2], e[3]),
-                        cvt_pk_bf16(e[4], e[5]), cvt_pk_bf16(e[6], e[7])));
-                }
+                for (int j = 0; j < 8; ++j) e[j] = __expf(e[j] - base);
+                p[n][c] = as_frag(make_uint4(
+                    cvt_pk_bf16(e[0], e[1]), cvt_pk_bf16(e[2], e[3]),
+                    cvt_pk_bf16(e[4], e[5]), cvt_pk_bf16(e[6], e[7])));
             }
-            l[n] += sum;
+            l[n] = fmaf(l[n], factor[n], pf_key_sum(s[n]));
         }
 
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
-            const int at = value_at + ((d ^ (v_row & 7)) << 5);
+            const int at = value_at + ((d ^ ((v_row & 3) | (v_row >> 3 & 1) << 2)) << 5);
 #pragma unroll
-            for (int c = 0; c < CHUNKS; ++c) {
+            for (int c = 0; c < 2; ++c) {
                 const bf16* lo = reinterpret_cast<const bf16*>(vals + at + c * 32 * PF_ROW);
-                const bf16x8 vf = tr_pair(lo, lo + 16 * PF_D);
+                const bf16x8 vf = tr_pair(lo, lo + 4 * PF_D);
 #pragma unroll
-                for (int n = 0; n < NQ; ++n) {
-                    acc[n][d] = mfma16(vf, p[n][c], acc[n][d]);
-                    if constexpr (FINE) acc[n][d] = mfma16(vf, p_low[n][c], acc[n][d]);
-                }
+                for (int n = 0; n < NQ; ++n) acc[n][d] = mfma16(vf, p[n][c], acc[n][d]);
             }
         }
     }
@@ -353,10 +385,9 @@ __global__ void attention_prefill_kernel(
     if (!has_head) return;
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
-        const float sum = pf_column_sum(l[n]);
         const int r = row0 + n * 16 + col;
-        if (r >= seq_len || sum <= 0.f) continue;
-        const float inv = 1.f / sum;
+        if (r >= seq_len || l[n] <= 0.f) continue;
+        const float inv = 1.f / l[n];
         bf16* o = out + ((int64_t)(seq_start + r) * Hq + head) * PF_D + grp * 4;
 #pragma unroll
         for (int d = 0; d < 8; ++d)
@@ -378,23 +409,21 @@ extern "C" hipError_t launch_attention_prefill(
     if (Hkv <= 0 || Hq % Hkv != 0) return hipErrorInvalidValue;
     if (ntiles <= 0) return hipSuccess;
     const int G = Hq / Hkv;
-    const float c = fmaxf(fabsf(scale) * 1.44269504088896f, 1e-30f);
-    const uint32_t q_sign = scale < 0.f ? 0x80008000u : 0u;
-#define LAUNCH(HG, KT, FINE)                                                       \
+#define LAUNCH(HG)                                                       \
     do {                                                                       \
         const int groups = (G + HG - 1) / HG;                                  \
         const dim3 grid(Hkv * groups * ntiles), block(HG * 2 * WAVE_SIZE);      \
         if (k_scale != nullptr)                                                \
-            attention_prefill_kernel<HG, KT, true, FINE><<<grid, block, 0, stream>>>(\
+            attention_prefill_kernel<HG, true><<<grid, block, 0, stream>>>(\
                 (bf16*)out, (const bf16*)q, (const bf16*)k, (const bf16*)v,    \
-                cu_seqlens, tile_seq, tile_off, c, q_sign, G, Hkv, groups,     \
+                cu_seqlens, tile_seq, tile_off, scale, G, Hkv, groups,     \
                 q_stride, k_stride, v_stride, (const char*)k_cache,            \
                 (const char*)v_cache, k_scale, v_scale, block_tables,          \
                 cached_lens, block_size, max_blocks);                          \
         else                                                                   \
-            attention_prefill_kernel<HG, KT, false, FINE><<<grid, block, 0, stream>>>(\
+            attention_prefill_kernel<HG, false><<<grid, block, 0, stream>>>(\
                 (bf16*)out, (const bf16*)q, (const bf16*)k, (const bf16*)v,    \
-                cu_seqlens, tile_seq, tile_off, c, q_sign, G, Hkv, groups,     \
+                cu_seqlens, tile_seq, tile_off, scale, G, Hkv, groups,     \
                 q_stride, k_stride, v_stride, (const char*)k_cache,            \
                 (const char*)v_cache, k_scale, v_scale, block_tables,          \
                 cached_lens, block_size, max_blocks);                          \
@@ -402,20 +431,16 @@ extern "C" hipError_t launch_attention_prefill(
     // Heads of a workgroup, by how many workgroups of four heads there would be.
     // Four (three where that divides the group better) where they fill the 256
     // CUs; two where CUs would idle, or where sequences are short and latency
-    // counts; one, and half the keys a tile, for a tile or two. 32:8 heads, us
-    // with 4 / 2 / 1 heads: 4096 tokens 158 / 166 / 192, 9 x 117-213 after 1984
-    // 90 / 99 / 133, 1000 tokens 37 / 29 / 37, 32 x 66-128 26 / 23 / 23, 300
-    // tokens 16 / 12 / 13, 37 tokens 7.8 / 6.0 / 5.1. One head a kv head: keys
-    // are used once, 4096 tokens take 202 us with 32 a tile, 233 with 64.
+    // counts. 32:8 heads, us with 4 / 2 / 1 heads: 4096 tokens 189 / 199 / 329, 9 x
+    // 117-213 after 1984 106 / 110 / 231, 1000 tokens 44 / 34 / 44, 32 x 66-128 27 /
+    // 24 / 35, 300 tokens 18 / 13 / 16, 37 tokens 7.9 / 6.6 / 7.2. One head a kv
+    // head: the waves without one bring keys (32 heads, 2000 tokens 89 us with two,
+    // 93 with one; 150 tokens after 1000 46 and 66).
     const int full = ntiles * Hkv * ((G + 3) / 4);
     const bool short_keys = cached_lens == nullptr && ntiles <= 4 * nseq;
-    // A tile or two also have their weights in 16 bits of mantissa: it costs 0.3
-    // us there, and a short prompt gives what decoding over it gives.
-    if (full <= 16) LAUNCH(1, 32, true);
-    else if (G == 1) LAUNCH(1, 32, false);
-    else if (G == 2 || full < 160 || short_keys) LAUNCH(2, 64, false);
-    else if (G == 3 || G == 5 || G == 6) LAUNCH(3, 64, false);
-    else LAUNCH(4, 64, false);
+    if (G <= 2 || full < 160 || short_keys) LAUNCH(2);
+    else if (G == 3 || G == 5 || G == 6) LAUNCH(3);
+    else LAUNCH(4);
 #undef LAUNCH
     HIP_CHECK_LAST();
     return hipSuccess;

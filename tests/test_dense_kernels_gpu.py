@@ -158,6 +158,88 @@ def test_attention_prefill_edges(lens, cached, Hkv, G, BS, fp8):
             torch.testing.assert_close(got[at, h].double(), ref, rtol=2**-8, atol=atol)
 
 
+def _prompt_attention_in_order(q, k, v, cached):
+    """[n, D] of one head over keys [cached + n, D]: 64 keys at a time (the cached
+    ones apart), scores in fp32 relative to the largest so far, weights in bf16
+    for the values and in fp32 for their sum."""
+    n = q.shape[0]
+    m = torch.full((n, 1), -math.inf, device=DEV)
+    l = torch.zeros(n, 1, device=DEV)
+    acc = torch.zeros(n, D, dtype=torch.float64, device=DEV)
+    row = torch.arange(n, device=DEV).unsqueeze(1)
+    for at in (*range(0, cached, 64), *range(cached, cached + n, 64)):
+        end = min(at + 64, cached if at < cached else cached + n)
+        s = (q.double() @ k[at:end].double().T).float() * torch.tensor(D**-0.5, device=DEV)
+        s = s.masked_fill(torch.arange(at, end, device=DEV) > row + cached, -math.inf)
+        top = torch.maximum(m, s.amax(-1, keepdim=True))
+        w, factor = (s - top).exp(), (m - top).exp()
+        l = l * factor + w.sum(-1, keepdim=True)
+        acc = acc * factor.double() + w.bfloat16().double() @ v[at:end].double()
+        m = top
+    return (acc / l.double()).bfloat16()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize(
+    "n,cached,Hkv,G",
+    [(37, 0, 2, 4), (300, 0, 2, 4), (130, 0, 4, 1), (200, 500, 2, 7), (257, 129, 1, 5),
+     (700, 64, 8, 4), (65, 31, 1, 6)],
+)
+def test_attention_prefill_order(n, cached, Hkv, G, fp8):
+    """However heads are shared out, sums are in the order above: but for the last
+    bit of fp32 sums, which shows in few roundings to bf16, the same comes out."""
+    if fp8 and not cached:
+        pytest.skip("no pages, no bytes")
+    torch.manual_seed(n + cached)
+    q, k, v = ((torch.randn(n, h, D, device=DEV) * 1.3).bfloat16() for h in (Hkv * G, Hkv, Hkv))
+    more, keys = {}, [k.transpose(0, 1), v.transpose(0, 1)]
+    if cached:
+        kv, scales, wide, tables = _pages([cached], Hkv, 64, fp8, n)
+        more = dict(
+            k_cache=kv[0], v_cache=kv[1], block_tables=tables,
+            cached_lens=torch.tensor([cached], dtype=torch.int32, device=DEV),
+            k_scale=scales[0], v_scale=scales[1],
+        )
+        pages = (x[tables[0].long()].transpose(0, 1).reshape(Hkv, -1, D)[:, :cached] for x in wide)
+        keys = [torch.cat([a.float().bfloat16(), b], 1) for a, b in zip(pages, keys)]
+    cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    got = ops.attention_prefill(q, k, v, cu, n, **more)
+    want = torch.stack([
+        _prompt_attention_in_order(q[:, h], keys[0][h // G], keys[1][h // G], cached)
+        for h in range(Hkv * G)
+    ], 1)
+    # fp32 sums and exponentials are off by some 2^-22, so of the weights, 2^-8 of
+    # themselves apart, one in 2^13 rounds to its neighbour: a result changes by
+    # 2^-8 of one weight in thousands, or 2^-22 by its own sum, and rounds to its
+    # neighbour in a percent of cases. Weights that are relative to anything but
+    # the largest so far turn a fifth and more.
+    differ = float((got != want).double().mean())
+    assert differ < 0.02, differ
+
+
+# behind the last key a tile has its row again, with weights of 0
+@pytest.mark.parametrize("cached", [0, 70])
+def test_attention_prefill_infinite_values(cached):
+    torch.manual_seed(5)
+    n, Hkv, G = 70, 2, 2
+    q, k, v = (torch.randn(n, h, D, device=DEV).bfloat16() for h in (Hkv * G, Hkv, Hkv))
+    more = {}
+    if cached:
+        kv, _, _, tables = _pages([cached], Hkv, 64, False, 3)
+        kv[1][tables[0, 1], 1, 5, 7] = -math.inf  # the last one
+        more = dict(
+            k_cache=kv[0], v_cache=kv[1], block_tables=tables,
+            cached_lens=torch.tensor([cached], dtype=torch.int32, device=DEV),
+        )
+    else:
+        v[-1, 1, 7] = -math.inf
+    cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    got = ops.attention_prefill(q, k, v, cu, n, **more)
+    sees = slice(None) if cached else slice(n - 1, None)
+    assert bool((got[sees, G:, 7] == -math.inf).all())
+    assert bool(got[:, :G].isfinite().all()) and bool(got[:64].isfinite().all() or cached)
+
+
 # rows that start off 16 bytes (odd V), shorter than the workgroup, more equal
 # tokens than the list of a coarse bin holds, masked and NaN tokens
 @pytest.mark.parametrize("V", [5, 63, 1000, 4097, 32003, 128256])

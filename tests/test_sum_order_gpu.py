@@ -81,3 +81,47 @@ def test_sum_parts_refuses():
     for args in ((y[:3], parts), (y, parts.double()), (y, parts[0]), (y[:, :32], parts)):
         with pytest.raises(RuntimeError):
             ops._native().sum_parts(*args)
+
+
+# the last layer's pages and scales after a step over prompts of up to 16 rows
+# (no library product among them), as separate kernels of slabs gave them
+@pytest.mark.parametrize(
+    "T,cached,bytes_,scales",
+    [(5, 0, 3593197530, 1828829798), (13, 0, 315290881, 461129092),
+     (16, 32, 3583420357, 2088370348)],
+)
+def test_prompt_bytes(T, cached, bytes_, scales):
+    from llmapigateway_amd.engine.kvcache import PagedKVCache
+    from llmapigateway_amd.models import build_model
+    from llmapigateway_amd.models.batch import ForwardBatch
+    from llmapigateway_amd.models.configs import ModelConfig
+
+    c = ModelConfig(
+        name="bytes", hidden_size=2048, intermediate_size=1024, num_layers=4, num_heads=4,
+        num_kv_heads=2, vocab_size=2048, head_dim=128, rope_theta=10000.0, max_positions=1024,
+    )
+    model = build_model(c, device=DEV, dtype=torch.bfloat16, seed=3)
+    cache = PagedKVCache(c, 8, 16, DEV, torch.bfloat16, kv_dtype="fp8")
+    rs = np.random.RandomState(T)
+    for pages, scale in zip(cache.k_caches + cache.v_caches, cache.k_scales + cache.v_scales):
+        pages.copy_(_rows(rs, *pages.shape, by=64).float().to(torch.float8_e4m3fn).view(torch.uint8))
+        scale.fill_(0.02)
+    order = torch.tensor([5, 0, 7, 2], device=DEV)
+    n = torch.arange(cached, cached + T, device=DEV)
+    more = {}
+    if cached:
+        more = dict(
+            block_tables=order.int().unsqueeze(0),
+            cached_lens=torch.tensor([cached], dtype=torch.int32, device=DEV),
+        )
+    tile_seq, tile_off = ops.build_prefill_tiles([T], torch.device(DEV))
+    batch = ForwardBatch(
+        kind="prefill", token_ids=n * 7 % 2048, positions=n, slot_mapping=order[n // 16] * 16 + n % 16,
+        cu_seqlens=torch.tensor([0, T], dtype=torch.int32, device=DEV), max_seqlen=T,
+        tile_seq=tile_seq, tile_off=tile_off,
+        logits_indices=torch.tensor([T - 1], device=DEV), **more,
+    )
+    model.step(batch, cache)
+    got = (_crc(torch.stack([cache.k_caches[-1], cache.v_caches[-1]])),
+           _crc(torch.stack([cache.k_scales[-1], cache.v_scales[-1]])))
+    assert got == (bytes_, scales), got
