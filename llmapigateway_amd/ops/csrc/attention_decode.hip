@@ -414,6 +414,25 @@ __global__ void attention_decode_kernel(
 #pragma unroll
             for (int r = 0; r < 4; ++r) o[r] += f * a[r];
         }
+        // 0 times an infinity, as the low half of a weight or that of a row behind
+        // the last key, is not what the sum of weights and values has there
+        if (!FP8 && gl == gl && !(o[0] - o[0] + o[1] - o[1] + o[2] - o[2] + o[3] - o[3] == 0.f)) {
+            float odd[4] = {0.f, 0.f, 0.f, 0.f};
+            for (int key = start; key < stop; ++key) {
+                const int64_t at = ((int64_t)table[key / block_size] * Hkv + kvh) * block_size +
+                                   key % block_size;
+                const uint2 raw = *reinterpret_cast<const uint2*>(v_cache + at * Tile::ROW + d * 2);
+                float v[4];
+                unpack2(raw.x, v[0], v[1]);
+                unpack2(raw.y, v[2], v[3]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (v[r] - v[r] != 0.f) odd[r] += v[r];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (odd[r] != 0.f) o[r] = odd[r];
+        }
         const size_t row = (size_t)seq * Hkv * G + kvh * G + g;
         if (SPLIT) {
             const size_t pb = row * nsplit + split;

@@ -80,6 +80,28 @@ def test_attention_decode_edges(lens, Hkv, G, BS, most, fp8):
         torch.testing.assert_close(got[b].double(), ref, rtol=2**-8, atol=1e-4)
 
 
+# an infinite value stays one, at the last key (whose row fills up its tile) and
+# elsewhere, with one sign and both; a NaN, too
+@pytest.mark.parametrize("B,most", [(3, 4096), (60, None)])
+@pytest.mark.parametrize("at", [0, 33, 99])
+def test_attention_decode_infinite_values(B, most, at):
+    kv, _, _, tables = _pages([100] * B, 4, 16, False, B, most)
+    v, dims = kv[1], {3: math.inf, 60: -math.inf, 101: math.nan}
+    for d, x in dims.items():
+        v[tables[1, at // 16], 2, at % 16, d] = x
+    v[tables[1, 1], 2, 5, 7], v[tables[1, 4], 2, 5, 7] = math.inf, -math.inf
+    q = torch.randn(B, 8, D, device=DEV).bfloat16() * 0.1
+    ctx = torch.full((B,), 100, dtype=torch.int32, device=DEV)
+    got = ops.attention_decode(q, *kv, tables, ctx)
+    rows = got[1, 4:6]
+    assert bool((rows[:, 3] == math.inf).all()) and bool((rows[:, 60] == -math.inf).all())
+    assert bool(rows[:, [7, 101]].isnan().all())
+    assert int((~got.isfinite()).sum()) == 8
+    # scores that are not numbers leave none
+    kv[0][tables[1, 0], 2, 1, 9] = math.nan
+    assert bool(ops.attention_decode(q, *kv, tables, ctx)[1, 4:6].isnan().all())
+
+
 # pages that the context before or behind has too are read another way than
 # others: the same values come out
 @pytest.mark.parametrize("fp8", [False, True])
