@@ -323,6 +323,9 @@ class LLMEngine:
             raise ValueError(
                 f"Prompt of {len(req.prompt_ids)} tokens exceeds max_model_len={self.max_model_len}"
             )
+        vocab = self.full_config.vocab_size
+        if req.prompt_ids and not 0 <= min(req.prompt_ids) <= max(req.prompt_ids) < vocab:
+            raise ValueError(f"Prompt holds a token id outside the vocabulary of {vocab}")
         with self._work:
             req.enqueued = time.monotonic()
             self.waiting.append(req)

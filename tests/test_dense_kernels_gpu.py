@@ -578,6 +578,18 @@ def test_embed_rows(T, H):
     assert none is None and torch.equal(again, r)
 
 
+@pytest.mark.parametrize("H", [512, 4096])
+def test_embed_rows_unknown_tokens(H):
+    embed = torch.randn(70, H, device=DEV).bfloat16()
+    w = torch.ones(H, device=DEV).bfloat16()
+    tokens = torch.tensor([3, -1, 69, 70, 2**40], device=DEV)
+    for normed in (False, True):
+        r, x = ops.embed_rows(tokens, embed, w, 1e-5, normed=normed)
+        assert torch.equal(r[::2][:2], embed[[3, 69]])
+        for rows in (r, x) if normed else (r,):
+            assert bool(rows[[1, 3, 4]].isnan().all()) and bool(rows[[0, 2]].isfinite().all())
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 def test_tiled_steps_match_others(fp8, monkeypatch):
     """A step whose products go to gemm_tile (of 9 and 20 rows to gemm_stream) and the

@@ -128,6 +128,16 @@ def test_prompt_too_long_rejected():
         eng.add_request(EngineRequest(list(range(20)), SamplingParams()))
 
 
+@pytest.mark.parametrize("ids", [[1, -1], [512], [3, 2**40, 4]])
+def test_unknown_token_rejected(ids):
+    eng = make_engine()
+    assert eng.config.vocab_size == 512
+    with pytest.raises(ValueError):
+        eng.add_request(EngineRequest(ids, SamplingParams()))
+    assert not eng.has_work()
+    eng.add_request(EngineRequest([0, 511], SamplingParams(max_tokens=1)))
+
+
 def test_on_token_callbacks():
     eng = make_engine()
     seen = []
