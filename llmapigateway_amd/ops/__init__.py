@@ -725,7 +725,7 @@ def norm_logits(
     r: torch.Tensor, norm: torch.Tensor, eps: float, w: torch.Tensor
 ) -> torch.Tensor:
     """rmsnorm(r) @ w.T in fp32."""
-    return logits_linear(rmsnorm(r, norm, eps), w)
+    return logits_linear(rmsnorm(r, norm, eps) if r.shape[0] else r, w)
 
 
 # A batch's rows have the products in tiles (csrc/gemm_tile.hip), K split over

@@ -464,6 +464,36 @@ def test_streamed_steps_match_others():
     assert float(diff) < 0.02, float(diff)
 
 
+@pytest.mark.parametrize("T", [4, 40, 600])
+def test_steps_without_logits(T):
+    """A step that asks for no row's logits gets none, by few rows, tiles and
+    separate kernels."""
+    from llmapigateway_amd.engine.kvcache import PagedKVCache
+    from llmapigateway_amd.models import build_model
+    from llmapigateway_amd.models.batch import ForwardBatch
+    from llmapigateway_amd.models.configs import ModelConfig
+
+    c = ModelConfig(
+        name="rows", hidden_size=2048, intermediate_size=1024, num_layers=1, num_heads=4,
+        num_kv_heads=2, vocab_size=2048, head_dim=128, rope_theta=10000.0, max_positions=1024,
+    )
+    model = build_model(c, device=DEV, dtype=torch.bfloat16, seed=3)
+    cache = PagedKVCache(c, 40, 16, DEV, torch.bfloat16)
+    n = torch.arange(T, device=DEV)
+    tile_seq, tile_off = ops.build_prefill_tiles([T], torch.device(DEV))
+    batch = ForwardBatch(
+        kind="prefill", token_ids=n, positions=n, slot_mapping=n,
+        cu_seqlens=torch.tensor([0, T], dtype=torch.int32, device=DEV), max_seqlen=T,
+        tile_seq=tile_seq, tile_off=tile_off,
+        logits_indices=torch.zeros(0, dtype=torch.long, device=DEV),
+    )
+    got = model.step(batch, cache)
+    assert got.shape == (0, 2048) and got.dtype == torch.float32
+    # the rows are in their pages all the same
+    pages = cache.k_caches[0].transpose(1, 2).reshape(-1, 2 * D)
+    assert bool((pages[:T] != 0).any(1).all()) and bool((pages[T:] == 0).all())
+
+
 # tiles of 64, 128 and 256 rows, of 64 to 256 columns; one tile of depth and
 # more splits than there are; columns and rows that end inside a tile
 @pytest.mark.parametrize("M", [1, 17, 64, 65, 128, 129, 200, 256, 257, 385, 512])
