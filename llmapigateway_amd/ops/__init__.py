@@ -648,6 +648,7 @@ def embed_rows(
         embed.is_cuda and embed.dtype == torch.bfloat16 and embed.is_contiguous()
         and embed.data_ptr() % 16 == 0 and tokens.numel() > 0 and tokens.dim() == 1
         and tokens.dtype == torch.long and tokens.is_contiguous()
+        and embed.shape[1] % 8 == 0 and embed.shape[1] <= 16384  # what a workgroup holds
     ):
         r = torch.empty(
             (tokens.shape[0], embed.shape[1]), dtype=embed.dtype, device=embed.device

@@ -43,7 +43,8 @@ float* scale_ptr(const c10::optional<torch::Tensor>& s) {
     return s->data_ptr<float>();
 }
 
-// Attention reads rows 16 bytes at a time: what lies otherwise is copied.
+// Attention reads rows, others norms' weights 16 bytes at a time: what lies
+// otherwise is copied.
 torch::Tensor aligned(const torch::Tensor& t) {
     const int64_t each = 16 / t.element_size();
     bool fits = reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
@@ -320,10 +321,12 @@ void gemm_stream_rows(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t
     const int M = x.size(0), K = x.size(1), N = w.size(0);
     TORCH_CHECK(w.size(1) == K && y.size(0) == M && y.size(1) == (leaves == 1 ? N / 2 : N));
     const void* np = nullptr;
+    torch::Tensor weight;
     if (norm.has_value() && norm->defined()) {
         check_bf16(*norm, "norm");
-        TORCH_CHECK(dense16(*norm) && norm->numel() == K);
-        np = norm->data_ptr();
+        TORCH_CHECK(norm->is_contiguous() && norm->numel() == K);
+        weight = aligned(*norm);
+        np = weight.data_ptr();
     }
     CHECK_HIP(launch_gemm_stream(y.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, (int)leaves,
                                  np, (float)eps, current_stream()));
@@ -365,10 +368,11 @@ void add_parts_norm(torch::Tensor out, torch::Tensor r, torch::Tensor parts,
     check_bf16(weight, "weight");
     TORCH_CHECK(r.dim() == 2 && parts.dim() == 3 && parts.scalar_type() == torch::kFloat32 &&
                 parts.is_cuda());
-    TORCH_CHECK(dense16(out) && dense16(r) && dense16(weight) && dense16(parts));
+    TORCH_CHECK(dense16(out) && dense16(r) && weight.is_contiguous() && dense16(parts));
     const int T = r.size(0), H = r.size(1);
     TORCH_CHECK(out.sizes() == r.sizes() && weight.numel() == H && parts.size(1) == T &&
                 parts.size(2) == H);
+    weight = aligned(weight);
     CHECK_HIP(launch_add_parts_norm(out.data_ptr(), r.data_ptr(), parts.data_ptr<float>(),
                                     weight.data_ptr(), (float)eps, T, H, (int)parts.size(0),
                                     current_stream()));
@@ -381,7 +385,8 @@ void embed_norm(c10::optional<torch::Tensor> out, torch::Tensor r, torch::Tensor
     check_bf16(embed, "embed");
     check_bf16(weight, "weight");
     TORCH_CHECK(r.dim() == 2 && embed.dim() == 2 && dense16(r) && dense16(embed) &&
-                dense16(weight));
+                weight.is_contiguous());
+    weight = aligned(weight);
     const int T = r.size(0), H = r.size(1);
     TORCH_CHECK(tokens.is_cuda() && tokens.scalar_type() == torch::kInt64 &&
                 tokens.is_contiguous() && tokens.numel() == T);
@@ -449,7 +454,8 @@ void gemm_stream_qkv(torch::Tensor y, torch::Tensor x, torch::Tensor w, torch::T
     check_bf16(k_cache, "k_cache");
     check_bf16(v_cache, "v_cache");
     TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && y.dim() == 2 && k_cache.dim() == 4);
-    TORCH_CHECK(dense16(x) && dense16(w) && dense16(norm) && y.is_contiguous());
+    TORCH_CHECK(dense16(x) && dense16(w) && norm.is_contiguous() && y.is_contiguous());
+    norm = aligned(norm);
     TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() &&
                 v_cache.sizes() == k_cache.sizes());
     TORCH_CHECK(positions.scalar_type() == torch::kInt64 && positions.is_contiguous());

@@ -464,6 +464,48 @@ def test_streamed_steps_match_others():
     assert float(diff) < 0.02, float(diff)
 
 
+@pytest.mark.parametrize("H", [4, 12, 16392])
+def test_embed_rows_of_other_sizes(H):
+    """What the kernel does not hold is gathered."""
+    embed = torch.randn(70, H, device=DEV).bfloat16()
+    tokens = torch.randint(0, 70, (9,), device=DEV)
+    r, x = ops.embed_rows(tokens, embed, torch.ones(H, device=DEV).bfloat16(), 1e-5, normed=False)
+    assert x is None and torch.equal(r, embed[tokens])
+
+
+@pytest.mark.parametrize("T", [4, 40])
+def test_norm_weights_off_16_bytes(T):
+    """Layers whose norms' weights are views that start anywhere, by few rows and
+    tiles: as with weights that lie alone."""
+    from llmapigateway_amd.engine.kvcache import PagedKVCache
+    from llmapigateway_amd.models import build_model
+    from llmapigateway_amd.models.batch import ForwardBatch
+    from llmapigateway_amd.models.configs import ModelConfig
+
+    c = ModelConfig(
+        name="rows", hidden_size=2048, intermediate_size=1024, num_layers=2, num_heads=4,
+        num_kv_heads=2, vocab_size=2048, head_dim=128, rope_theta=10000.0, max_positions=1024,
+    )
+    model = build_model(c, device=DEV, dtype=torch.bfloat16, seed=3)
+
+    def off(w):
+        return torch.cat([w.new_zeros(1), w])[1:]
+
+    n = torch.arange(T, device=DEV)
+    logits = []
+    for kv in ("auto", "fp8"):
+        for _ in range(2):
+            cache = PagedKVCache(c, 40, 16, DEV, torch.bfloat16, kv_dtype=kv)
+            logits.append(model.step(ForwardBatch(
+                kind="decode", token_ids=n, positions=n % 16, slot_mapping=n * 16 + n % 16,
+                block_tables=n.int().unsqueeze(1).contiguous(), context_lens=(n % 16 + 1).int(),
+            ), cache))
+            for layer in model.layers:
+                layer.update({k: off(layer[k]) for k in ("input_norm", "post_norm")})
+            model.final_norm = off(model.final_norm)
+        assert torch.equal(*logits[-2:])
+
+
 @pytest.mark.parametrize("T", [4, 40, 600])
 def test_steps_without_logits(T):
     """A step that asks for no row's logits gets none, by few rows, tiles and
