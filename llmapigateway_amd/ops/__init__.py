@@ -473,10 +473,12 @@ def _streams_swiglu(M: int, N: int) -> bool:
 
 
 def _streamable(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """What gemm_stream asks of its operands."""
+    """What gemm_stream asks of its operands; it has no derivative."""
     return (
         x.is_cuda and x.dim() == 2 and x.shape[0] > 0
+        and w.numel() > 0 and w.shape[1] < 2**25
         and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+        and not ((x.requires_grad or w.requires_grad) and torch.is_grad_enabled())
         and x.is_contiguous() and w.is_contiguous()
         and w.shape[0] % 64 == 0 and w.shape[1] % 32 == 0
         and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0

@@ -379,6 +379,25 @@ def test_gemm_stream_refuses():
     assert ops.linear(x[:4], off).shape == (4, 64)
 
 
+def test_linear_of_other_operands():
+    """What gemm_stream does not take goes where it went: products to be derived,
+    without columns or depth."""
+    x = torch.randn(32, 64, device=DEV).bfloat16()
+    w = torch.randn(128, 64, device=DEV).bfloat16()
+    for a, b in ((x.clone().requires_grad_(), w), (x, w.clone().requires_grad_())):
+        ops.linear(a, b).float().sum().backward()
+        wide = [t.detach().float().requires_grad_(t.requires_grad) for t in (a, b)]
+        torch.nn.functional.linear(*wide).sum().backward()
+        for t, u in zip((a, b), wide):
+            if t.requires_grad:
+                torch.testing.assert_close(t.grad.float(), u.grad, rtol=2**-7, atol=2**-5)
+    with torch.no_grad():
+        got = ops.linear(x.clone().requires_grad_(), w)
+    assert torch.equal(got, ops.linear(x, w))
+    assert ops.linear(x, w[:0]).shape == (32, 0)
+    assert bool((ops.linear(x[:, :0], w[:, :0]) == 0).all())
+
+
 # a block of 16 rows and two, tiles that end inside a row, few and many column
 # blocks; against float64 from the same bf16 stream
 @pytest.mark.parametrize("T", [1, 5, 16, 17, 32])
