@@ -624,7 +624,7 @@ def layer_streams(T: int, layer: dict) -> bool:
     are ahead for large layers (32 rows of hidden size 4096: 110 us a layer
     streamed, 105 tiled; of 3584: 120 and 109), for smaller ones the fewer
     launches (3072: 60 and 66; 2048: 43 and 44)."""
-    if not 0 < T <= 32 or os.environ.get("LLMAPI_NO_FUSED_SWIGLU"):
+    if not 0 < T <= 32:
         return False
     qkv, o, gate_up, down = weights = [layer[k] for k in ("qkv", "o", "gate_up", "down")]
     return (
@@ -709,6 +709,8 @@ def norm_swiglu_linear(
     r: torch.Tensor, norm: torch.Tensor, eps: float, w: torch.Tensor
 ) -> torch.Tensor:
     """swiglu(rmsnorm(r) @ w.T), w = [gate; up] stacked."""
+    if r.is_cuda and os.environ.get("LLMAPI_NO_FUSED_SWIGLU"):
+        return swiglu(linear(rmsnorm(r, norm, eps), w))
     if r.is_cuda:
         y = torch.empty((r.shape[0], w.shape[0] // 2), dtype=r.dtype, device=r.device)
         _native().gemm_stream_rows(y, r, w, 1, norm, eps)
@@ -755,7 +757,6 @@ def layer_tiles(T: int, layer: dict, head_dim: int) -> bool:
     return (
         (8 if hidden < 8192 else 0) < T <= 512 and head_dim == 128
         and (1024 if T <= 128 else 2048) <= hidden <= 16384  # what add_parts_norm holds
-        and not os.environ.get("LLMAPI_NO_FUSED_SWIGLU")
         and all(_tileable(layer[k]) for k in ("qkv", "o", "gate_up", "down"))
         and not any(k.endswith("_swz") and w.dim() == 3 for k, w in layer.items())
     )
@@ -852,7 +853,10 @@ def _tiles_wide(M: int, N: int, K: int) -> bool:
 
 def swiglu_tiled(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """swiglu(x @ w.T), w = [gate; up] stacked."""
-    if x.is_cuda and _tiles_wide(x.shape[0], *w.shape):
+    if (
+        x.is_cuda and _tiles_wide(x.shape[0], *w.shape)
+        and not os.environ.get("LLMAPI_NO_FUSED_SWIGLU")
+    ):
         y = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype, device=x.device)
         _native().gemm_tile(y, x, w)
         return y

@@ -483,6 +483,39 @@ def test_streamed_steps_match_others():
     assert float(diff) < 0.02, float(diff)
 
 
+@pytest.mark.parametrize("T", [4, 40])
+def test_fused_swiglu_switch(T, monkeypatch):
+    """LLMAPI_NO_FUSED_SWIGLU takes swiglu apart from its product, of few rows and
+    of tiles, and leaves the rest of the layer as it is."""
+    from llmapigateway_amd.engine.kvcache import PagedKVCache
+    from llmapigateway_amd.models import build_model
+    from llmapigateway_amd.models.batch import ForwardBatch
+    from llmapigateway_amd.models.configs import ModelConfig
+
+    c = ModelConfig(
+        name="rows", hidden_size=2048, intermediate_size=1024, num_layers=2, num_heads=4,
+        num_kv_heads=2, vocab_size=2048, head_dim=128, rope_theta=10000.0, max_positions=1024,
+    )
+    model = build_model(c, device=DEV, dtype=torch.bfloat16, seed=3)
+    n = torch.arange(T, device=DEV)
+    apart, calls = ops.swiglu, []
+    monkeypatch.setattr(ops, "swiglu", lambda x: calls.append(x.shape) or apart(x))
+    routes, logits = [], []
+    for switch in ("", "1"):
+        monkeypatch.setenv("LLMAPI_NO_FUSED_SWIGLU", switch)
+        first = model.layers[0]
+        routes.append((ops.layer_streams(T, first), ops.layer_tiles(T, first, 128)))
+        cache = PagedKVCache(c, 40, 16, DEV, torch.bfloat16)
+        logits.append(model.step(ForwardBatch(
+            kind="decode", token_ids=n, positions=n % 16, slot_mapping=n * 16 + n % 16,
+            block_tables=n.int().unsqueeze(1).contiguous(), context_lens=(n % 16 + 1).int(),
+        ), cache))
+        assert len(calls) == (2 if switch else 0)
+    assert routes[0] == routes[1] and any(routes[0])
+    diff = (logits[0] - logits[1]).norm() / logits[0].norm()
+    assert float(diff) < 0.02, float(diff)  # two layers, each of whose ten roundings is 2^-9
+
+
 @pytest.mark.parametrize("H", [4, 12, 16392])
 def test_embed_rows_of_other_sizes(H):
     """What the kernel does not hold is gathered."""
