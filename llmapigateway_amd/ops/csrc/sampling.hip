@@ -158,11 +158,19 @@ __global__ void sample_combine_kernel(
 #define TPF_LIST 4096  // of a coarse bin's tokens, as a rule tens
 
 // A softmax mass relative to the row's largest, e in [0, 1], as a multiple of
-// 2^-31. Sums of these do not depend on their order, and are closer than fp32
-// sums: 128256 of them are off by 1e-7 of the largest. LDS adds whole numbers
-// in one instruction (fp32 in a loop of compare-and-swap: 190 us a row).
-__device__ __forceinline__ uint32_t mass_of(float e) {
-    return (uint32_t)__builtin_rintf(e * 2147483648.f);
+// 1 / units (mass_units below; at most 2^42, so that the low half of a double
+// that is 2^52 more has it). Sums of these do not depend on their order, and are
+// as close as fp32 sums at least: up to 2^20 tokens round to 2^-43 each, 128256 of
+// them to 1.5e-8 together if all do so one way. LDS adds whole numbers in one
+// instruction (fp32 in a loop of compare-and-swap: 190 us a row). A NaN is none.
+__device__ __forceinline__ unsigned long long mass_of(float e, double units) {
+    return __double_as_longlong(fma((double)fmaxf(e, 0.f), units, 0x1p52)) & ((1ull << 52) - 1);
+}
+// 2^42, or what the sum over V tokens leaves room for
+static double mass_units(int V) {
+    double units = 0x1p42;
+    for (int64_t most = 1 << 20; most < V; most *= 2) units /= 2;
+    return units;
 }
 
 // f(value, its index) over a row of V floats, whose start need not be aligned
@@ -296,7 +304,8 @@ __device__ __forceinline__ unsigned long long block_sum(
 
 // the histogram of V values; returns, for a wave, NaN with any mass that is
 __device__ __forceinline__ float coarse_histogram(
-    float* row, int V, float m, bool do_k, bool do_p, int* cnt, unsigned long long* mass) {
+    float* row, int V, float m, double units, bool do_k, bool do_p, int* cnt,
+    unsigned long long* mass) {
     float nan = 0.f;
     auto histogram = [&](auto with_count, auto with_mass) {
         for_row<false>(row, V, [&](float& x, int) {
@@ -306,7 +315,7 @@ __device__ __forceinline__ float coarse_histogram(
             if constexpr (with_mass.value) {
                 const float e = __expf(-d);
                 nan += e;
-                atomicAdd(&mass[bin], (unsigned long long)mass_of(e));
+                atomicAdd(&mass[bin], mass_of(e, units));
             }
             return false;
         });
@@ -324,11 +333,12 @@ __device__ __forceinline__ unsigned long long mass_needed(
 }
 
 __device__ __forceinline__ void fine_count(
-    float d, int coarse, bool do_k, bool do_p, int* cnt, unsigned long long* mass) {
+    float d, int coarse, double units, bool do_k, bool do_p, int* cnt,
+    unsigned long long* mass) {
     const float d_lo = coarse / TPF_SCALE;  // the bin's lower edge (distance)
     const int fine = max(0, min((int)((d - d_lo) * (TPF_SCALE * TPF_BINS)), TPF_BINS - 1));
     if (do_k) atomicAdd(&cnt[fine], 1);
-    if (do_p) atomicAdd(&mass[fine], (unsigned long long)mass_of(__expf(-d)));
+    if (do_p) atomicAdd(&mass[fine], mass_of(__expf(-d), units));
 }
 
 // distances strictly below the fine bin's upper edge are kept
@@ -369,7 +379,7 @@ __global__ void topk_topp_filter_kernel(
     float* __restrict__ logits,          // [B, V], filtered in place
     const float* __restrict__ topp,      // [B]; >= 1 disables
     const int* __restrict__ topk,        // [B]; 0 disables
-    int V) {
+    int V, double units) {
     const int b = blockIdx.x;
     const float p = topp[b];
     const int k = topk[b];
@@ -399,7 +409,7 @@ __global__ void topk_topp_filter_kernel(
     m = block_max(m, s_red);
 
     // ---- pass 2: coarse histogram ----
-    float nan = coarse_histogram(row, V, m, do_k, do_p, s_cnt, s_mass);
+    float nan = coarse_histogram(row, V, m, units, do_k, do_p, s_cnt, s_mass);
     if ((tid & 63) == 0) s_nan[tid >> 6] = nan;
     __syncthreads();  // bins complete
     unsigned long long z = 0;  // all mass
@@ -427,7 +437,7 @@ __global__ void topk_topp_filter_kernel(
         const int bin = coarse_bin(d);  // of a NaN 0, in front of or in every other
         if (bin < coarse.bin) return false;
         if (bin == coarse.bin) {
-            fine_count(d, coarse.bin, do_k, do_p, s_cnt, s_mass);
+            fine_count(d, coarse.bin, units, do_k, do_p, s_cnt, s_mass);
             const int n = atomicAdd(&s_listed, 1);
             if (n < TPF_LIST) s_list[n] = at;
             return false;
@@ -462,6 +472,7 @@ struct FilterPieces {
     int* listed;               // [B]
     int* list;                 // [B, TPF_LIST]
     int pieces, V;
+    double units;
 
     __device__ __forceinline__ int first(int piece) const {
         const int each = ((V + pieces - 1) / pieces + 3) / 4 * 4;
@@ -512,7 +523,8 @@ __global__ void filter_coarse_kernel(
     __syncthreads();
     const int lo = f.first(piece);
     const float nan = coarse_histogram(
-        logits + (size_t)b * f.V + lo, f.first(piece + 1) - lo, m, do_k, do_p, s_cnt, s_mass);
+        logits + (size_t)b * f.V + lo, f.first(piece + 1) - lo, m, f.units, do_k, do_p, s_cnt,
+        s_mass);
     if ((tid & 63) == 0) s_red[tid >> 6] = nan;
     __syncthreads();
     const size_t at = (size_t)b * TPF_BINS;
@@ -600,7 +612,7 @@ __global__ void filter_fine_kernel(
     const int listed = f.listed[b];
     auto count = [&](float& x, int) {
         const float d = r.most - x;
-        if (coarse_bin(d) == r.bin) fine_count(d, r.bin, do_k, do_p, s_cnt, s_mass);
+        if (coarse_bin(d) == r.bin) fine_count(d, r.bin, f.units, do_k, do_p, s_cnt, s_mass);
         return false;
     };
     if (listed <= TPF_LIST) {
@@ -633,7 +645,8 @@ extern "C" hipError_t launch_topk_topp_filter(
     hipStream_t stream) {
     const int pieces = filter_pieces(B, V);
     if (pieces == 1) {
-        topk_topp_filter_kernel<<<B, TPF_THREADS, 0, stream>>>(logits, topp, topk, V);
+        topk_topp_filter_kernel<<<B, TPF_THREADS, 0, stream>>>(
+            logits, topp, topk, V, mass_units(V));
         HIP_CHECK_LAST();
         return hipSuccess;
     }
@@ -648,6 +661,7 @@ extern "C" hipError_t launch_topk_topp_filter(
     f.list = f.listed + B;
     f.pieces = pieces;
     f.V = V;
+    f.units = mass_units(V);
     const dim3 grid(B, pieces);
     filter_max_kernel<<<grid, TPF_THREADS, 0, stream>>>(logits, topp, topk, f);
     HIP_CHECK_LAST();

@@ -288,13 +288,28 @@ def test_topk_topp_filter_rows(V):
         least = ranked[int(keep.sum()) - 1] if bool(keep.any()) else ranked[0]
         kept = got[b] > -math.inf
         # what lies within the cut's granularity (16/2048^2) of it stays, too;
-        # masses are multiples of 2^-31 and exponentials good to 2^-22, so a
+        # masses are multiples of 2^-42 and exponentials good to 2^-22, so a
         # token may change sides where the mass in front of it is that close
         sure = x[b].double() >= least
         near = x[b].double() >= least - 4e-6
         extra = (kept & ~near).sum() + (sure & ~kept).sum()
         assert int(extra) <= (1 if topp[b] < 1 else 0), (V, b, int(extra))
         assert torch.equal(got[b][kept], x[b][kept])
+
+
+# many tokens of next to no mass, which together reach into what is asked for:
+# each is far below 2^-31 of the largest
+@pytest.mark.parametrize("V", [32000, 90000, 128256])
+@pytest.mark.parametrize("B", [1, 3, 70])
+def test_filter_counts_small_masses(V, B):
+    x = torch.full((B, V), -22.5, device=DEV)
+    x[:, V // 2] = 0.0
+    tail = math.exp(-22.5) * (V - 1)
+    topk = torch.zeros(B, dtype=torch.int32, device=DEV)
+    # the first token alone is enough up to 1 / (1 + tail), 4e-6 to 2e-5 below 1
+    for p, kept in ((1 - 1.5 * tail, 1), (1 - 0.5 * tail, V)):
+        got = ops.topk_topp_filter(x.clone(), torch.full((B,), p, device=DEV), topk)
+        assert ((got > -math.inf).sum(1) == kept).all(), (p, kept)
 
 
 # rows in 16, 5 and 4 pieces and whole ones: the same tokens stay
