@@ -468,6 +468,38 @@ def test_streamed_layer(T, H, Hq, Hkv, I):
         torch.testing.assert_close(got.double(), normed @ w.double().T, **near)
 
 
+# queries, keys and values of more than 8192 columns, additions to more than 4096:
+# workgroups of four waves
+@pytest.mark.parametrize("T", [1, 5, 16, 17, 32])
+@pytest.mark.parametrize("H,Hq,Hkv,I", [(4160, 56, 8, 256), (5120, 64, 2, 1024), (8192, 64, 8, 160)])
+def test_streamed_layer_wide(T, H, Hq, Hkv, I):
+    test_streamed_layer(T, H, Hq, Hkv, I)
+
+
+# what gemm_stream does not take of few rows: rows that end inside a tile, one
+# slab of K and several, operands that start anywhere
+@pytest.mark.parametrize("M", [1, 3, 15, 16])
+@pytest.mark.parametrize("N,K", [(64, 32), (192, 1056), (4096, 4096), (1024, 14336)])
+def test_gemm_skinny_rows(M, N, K):
+    g = torch.Generator(device=DEV).manual_seed(M * N + K)
+    x = torch.randn(M * K + 1, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N * K + 1, generator=g, device=DEV) / math.sqrt(K)).bfloat16()
+    # half a unit of bf16, and fp32 sums of K products of size 1/sqrt(K)
+    near = dict(rtol=2**-8, atol=2**-24 * K * float(x.abs().max()) * float(w.abs().max()))
+    for off in (0, 1):
+        a, b = x[off:][: M * K].view(M, K), w[off:][: N * K].view(N, K)
+        ref = a.double() @ b.double().T
+        nsk = ops._skinny_nsk(N, K)
+        assert nsk > 1 or K < 4096
+        ws = ops._skinny_scratch(x.device, nsk * M * N) if nsk > 1 else None
+        rows = torch.full((M + 2, N), 7.0, device=DEV).bfloat16()
+        ops._shared().gemm_skinny(rows[1:-1], a, b, ws, nsk, False)
+        torch.testing.assert_close(rows[1:-1].double(), ref, **near)
+        assert bool((rows[0] == 7).all()) and bool((rows[-1] == 7).all())
+        torch.testing.assert_close(ops.linear(a, b).double(), ref, **near)
+    assert not ops._streamable(a, b)
+
+
 def test_streamed_steps_match_others():
     """A step whose layers go to gemm_stream and the same step by separate
     kernels (a row more than they take, padded) agree to bf16's rounding."""
@@ -636,6 +668,13 @@ def test_gemm_tile_edges(M, N, K):
         torch.testing.assert_close(got, want, rtol=rtol, atol=atol * scale + (1e-5 if rtol else 0))
 
 
+# 16385 to 32768 columns: tiles of 128 of them
+@pytest.mark.parametrize("M", [1, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize("N,K", [(16416, 192), (28704, 64), (32768, 320)])
+def test_gemm_tile_wide(M, N, K):
+    test_gemm_tile_edges(M, N, K)
+
+
 def test_gemm_tile_refuses():
     def call(M, N, K, y, off=0):
         x = torch.zeros(M * K + off, device=DEV).bfloat16()[off:].view(M, K)
@@ -771,6 +810,93 @@ def test_tiled_steps_match_others(fp8, monkeypatch):
         # two layers, each of whose ten roundings is 2^-9; a row in e4m3 2^-4
         diff = (logits[0] - logits[1]).norm() / logits[1].norm()
         assert float(diff) < (0.05 if fp8 else 0.02), float(diff)
+
+
+def _steps_of(c, lens, cached, decodes, kv):
+    """A mixed step (of prompts alone where decodes is 0) and pages for it."""
+    from llmapigateway_amd.engine.kvcache import PagedKVCache
+    from llmapigateway_amd.models.batch import ForwardBatch
+
+    g = torch.Generator(device=DEV).manual_seed(sum(lens) + cached)
+    B, BS = len(lens) + decodes, 16
+    width = -(-(max(lens + [40]) + cached) // BS)
+    cache = PagedKVCache(c, B * width, BS, DEV, torch.bfloat16, kv_dtype=kv)
+    for pages, scale in zip(cache.k_caches + cache.v_caches,
+                            (cache.k_scales + cache.v_scales) if cache.fp8 else [None] * 99):
+        x = torch.randn(pages.shape, generator=g, device=DEV)
+        if cache.fp8:
+            pages.copy_((x * 64).to(torch.float8_e4m3fn).view(torch.uint8))
+            scale.fill_(0.02)
+        else:
+            pages.copy_(x)
+    tables = torch.randperm(B * width, generator=g, device=DEV).int().view(B, width)
+    context = torch.arange(decodes, device=DEV) % 40 + 1
+    positions = torch.cat(
+        [torch.arange(cached, cached + n, device=DEV) for n in lens] + [context - 1])
+    row = torch.tensor([i for i, n in enumerate(lens) for _ in range(n)], device=DEV)
+    row = torch.cat([row, torch.arange(len(lens), B, device=DEV)])
+    cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
+    tile_seq, tile_off = ops.build_prefill_tiles(lens, torch.device(DEV))
+    more = {}
+    if cached:
+        more.update(block_tables=tables[: len(lens)].contiguous(),
+                    cached_lens=torch.full((len(lens),), cached, dtype=torch.int32, device=DEV))
+    if decodes:
+        more.update(dec_block_tables=tables[len(lens):].contiguous(),
+                    dec_context_lens=context.int())
+    T = len(row)
+    return cache, ForwardBatch(
+        kind="mixed" if decodes else "prefill",
+        token_ids=torch.randint(0, c.vocab_size, (T,), generator=g, device=DEV),
+        positions=positions, slot_mapping=tables[row, positions // BS].long() * BS + positions % BS,
+        cu_seqlens=cu, max_seqlen=max(lens), tile_seq=tile_seq, tile_off=tile_off,
+        n_prefill_tokens=sum(lens),
+        logits_indices=torch.cat([cu[1:].long() - 1, torch.arange(sum(lens), T, device=DEV)]),
+        **more,
+    )
+
+
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize(
+    "lens,cached,decodes",
+    [([7], 0, 0), ([5, 3], 33, 4), ([11], 0, 21), ([40, 9], 0, 0), ([70, 1], 20, 30),
+     ([300], 0, 100), ([200, 57], 64, 3)],
+)
+def test_prompt_and_mixed_steps_match_others(lens, cached, decodes, kv, monkeypatch):
+    """Steps over prompts, with and without decoded rows beside them, by few rows
+    or tiles (e4m3: in order) and by separate kernels agree to bf16's rounding."""
+    from llmapigateway_amd.models import build_model
+    from llmapigateway_amd.models.configs import ModelConfig
+
+    c = ModelConfig(
+        name="rows", hidden_size=2048, intermediate_size=1024, num_layers=2, num_heads=4,
+        num_kv_heads=2, vocab_size=2048, head_dim=128, rope_theta=10000.0, max_positions=1024,
+    )
+    model = build_model(c, device=DEV, dtype=torch.bfloat16, seed=3)
+    got = []
+    T = sum(lens) + decodes
+    assert ops.layer_streams(T, model.layers[0]) or ops.layer_tiles(T, model.layers[0], 128)
+    for separate in (False, True):
+        if separate:
+            for route in ("layer_streams", "layer_tiles", "_streamable"):
+                monkeypatch.setattr(ops, route, lambda *a: False)
+            monkeypatch.setattr(
+                ops, "linear_in_order", lambda x, w, *a, **k: torch.nn.functional.linear(x, w))
+        cache, batch = _steps_of(c, lens, cached, decodes, kv)
+        logits = model.step(batch, cache)
+        assert logits.dtype == torch.float32 and logits.shape == (len(lens) + decodes, 2048)
+        rows = [logits]
+        for i, pages in enumerate(cache.k_caches + cache.v_caches):
+            x = pages
+            if cache.fp8:
+                scale = (cache.k_scales + cache.v_scales)[i]
+                x = pages.view(torch.float8_e4m3fn).float() * scale.unsqueeze(-1)
+            rows.append(x.transpose(1, 2).reshape(-1, 2 * D)[batch.slot_mapping].float())
+        got.append(rows)
+    for one, other in zip(*got):
+        # two layers, each of whose ten roundings is 2^-9; a row in e4m3 2^-4
+        diff = (one - other).norm() / other.norm()
+        assert float(diff) < (0.05 if kv == "fp8" else 0.02), float(diff)
 
 
 # a wave, 64 to 1024 threads a row, and pieces: the ends of each
