@@ -40,6 +40,10 @@
 
 #define DECODE_D 128
 #define MAX_G 8
+// four waves: with two a span of 900 keys takes 22.9 us instead of 16.7, with
+// eight 256 contexts of 192 take 44 us instead of 33; a third tile in the ring
+// gains nothing
+#define DECODE_WAVES 4
 #define MIN_SPAN 64  // keys of a workgroup's round (4 waves x 16)
 
 namespace {
@@ -71,33 +75,10 @@ struct DecodeTile {
     }
 };
 
-template <int N>
-__device__ __forceinline__ void wait_transfers() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // keys of one split of a context of length L
 __device__ __forceinline__ int span_of(int L, int nsplit) {
     const int even = (L + nsplit - 1) / nsplit;
     return (even + MIN_SPAN - 1) / MIN_SPAN * MIN_SPAN;
-}
-
-// maximum / sum over the four lanes that hold one column (l, l^16, l^32, l^48)
-__device__ __forceinline__ float column_max(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(
-        __float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(
-        __float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float column_sum(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(
-        __float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto b = __builtin_amdgcn_permlane32_swap(
-        __float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
 // 8 e4m3 bytes as 8 bf16 (exact)
@@ -121,8 +102,8 @@ __device__ __forceinline__ f32x4 mfma16_k16(bf16x4 a, bf16x4 b, f32x4 c) {
 // PAGED: pages hold whole tiles (block_size a multiple of the tile), so a tile
 // has one page; else every row looks its page up. SPLIT: partials instead of
 // the output.
-template <int W, int NB, bool FP8, bool SPLIT, bool PAGED>
-__launch_bounds__(W* WAVE_SIZE)
+template <bool FP8, bool SPLIT, bool PAGED>
+__launch_bounds__(DECODE_WAVES* WAVE_SIZE)
 __global__ void attention_decode_kernel(
     bf16* __restrict__ out,                // [B, Hq, D]
     const bf16* __restrict__ q,            // [B, Hq, D], rows q_stride apart
@@ -138,6 +119,7 @@ __global__ void attention_decode_kernel(
     float* __restrict__ part_ml,           // [B, Hq, nsplit, 2] (SPLIT)
     int nsplit) {
     using Tile = DecodeTile<FP8>;
+    constexpr int W = DECODE_WAVES, NB = 2;  // waves, and tiles of each in LDS
     const int seq = blockIdx.x, kvh = blockIdx.y, split = SPLIT ? blockIdx.z : 0;
     const int L = context_lens[seq];
     const int span = SPLIT ? span_of(L, nsplit) : L;
@@ -270,8 +252,7 @@ __global__ void attention_decode_kernel(
             if (fetched < mine) page = page_of(fetched);
         }
         const int ahead = fetched - 1 - i;
-        if (NB > 2 && ahead >= 2) wait_transfers<2 * Tile::IN_FLIGHT>();
-        else if (ahead >= 1) wait_transfers<Tile::IN_FLIGHT>();
+        if (ahead >= 1) wait_transfers<Tile::IN_FLIGHT>();
         else wait_transfers<0>();
 
         const char* keys = ring[wave][i % NB];
@@ -515,34 +496,22 @@ extern "C" hipError_t launch_attention_decode(
     const bool paged = block_size % (fp8 ? 32 : 16) == 0;
     const float scale_log2 = scale * 1.44269504088896f;
     const dim3 grid(B, Hkv, nsplit > 1 ? nsplit : 1);
-#define LAUNCH(W, NB, FP8, SPLIT, PAGED)                                       \
-    attention_decode_kernel<W, NB, FP8, SPLIT, PAGED>                          \
-        <<<grid, dim3(W * WAVE_SIZE), 0, stream>>>(                            \
+#define LAUNCH(FP8, SPLIT, PAGED)                                              \
+    attention_decode_kernel<FP8, SPLIT, PAGED>                                 \
+        <<<grid, dim3(DECODE_WAVES * WAVE_SIZE), 0, stream>>>(                 \
             (bf16*)out, (const bf16*)q, (const char*)k_cache,                  \
             (const char*)v_cache, k_scale, v_scale, block_tables,              \
             context_lens, scale_log2, Hkv, G, block_size, max_blocks,          \
             q_stride, part_acc, part_ml, nsplit)
-#define LAUNCH_P(W, NB, FP8, SPLIT)                                            \
+#define LAUNCH_P(FP8, SPLIT)                                                   \
     do {                                                                       \
-        if (paged) LAUNCH(W, NB, FP8, SPLIT, true);                            \
-        else LAUNCH(W, NB, FP8, SPLIT, false);                                 \
+        if (paged) LAUNCH(FP8, SPLIT, true);                                   \
+        else LAUNCH(FP8, SPLIT, false);                                        \
     } while (0)
-#define LAUNCH_S(W, NB, FP8)                                                   \
-    do {                                                                       \
-        if (nsplit > 1) LAUNCH_P(W, NB, FP8, true);                            \
-        else LAUNCH_P(W, NB, FP8, false);                                      \
-    } while (0)
-#define LAUNCH_F(W, NB)                                                        \
-    do {                                                                       \
-        if (fp8) LAUNCH_S(W, NB, true);                                        \
-        else LAUNCH_S(W, NB, false);                                           \
-    } while (0)
-    // four waves: with two a span of 900 keys takes 22.9 us instead of 16.7, with
-    // eight 256 contexts of 192 take 44 us instead of 33; a third tile in the
-    // ring gains nothing
-    LAUNCH_F(4, 2);
-#undef LAUNCH_F
-#undef LAUNCH_S
+    if (fp8 && nsplit > 1) LAUNCH_P(true, true);
+    else if (fp8) LAUNCH_P(true, false);
+    else if (nsplit > 1) LAUNCH_P(false, true);
+    else LAUNCH_P(false, false);
 #undef LAUNCH_P
 #undef LAUNCH
     HIP_CHECK_LAST();

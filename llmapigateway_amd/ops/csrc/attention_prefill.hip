@@ -56,14 +56,6 @@ __device__ __forceinline__ int pf_value_piece(int row, int p) {
     return (((p >> 1) ^ ((row & 3) | (row >> 3 & 1) << 2)) << 1) | (p & 1);
 }
 
-__device__ __forceinline__ float pf_column_max(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(
-        __float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(
-        __float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
 // The sum of 64 weights of one column, of which a lane has those of keys
 // 32c + 8*grp + 4h + r at [c][4h + r]: first the four of the keys that are equal
 // in their last 4 bits, in order, then these by halves (8 apart, 4, 2, 1). A swap
@@ -338,7 +330,7 @@ __global__ void attention_prefill_kernel(
             for (int c = 0; c < 2; ++c)
 #pragma unroll
                 for (int j = 0; j < 8; ++j) x = fmaxf(x, s[n][c][j]);
-            top[n] = pf_column_max(x);
+            top[n] = column_max(x);
         }
         float factor[NQ] = {1.f, 1.f};
         if (__any(top[0] > m[0] || top[1] > m[1])) {

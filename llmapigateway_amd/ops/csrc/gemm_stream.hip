@@ -6,8 +6,10 @@
 //   not in slabs of memory behind a second kernel.
 // - Each wave streams its tiles of W and X (rows of 128 or 256 bytes in a
 //   piece) through a ring of two in LDS by transfers that need no registers,
-//   waited for by count; no barrier before the sums meet. 64 KB of LDS a
-//   workgroup let two share a CU: 64 KB in flight there.
+//   waited for by count; no barrier before the sums meet. Rings of 53 to 82 KB
+//   let two workgroups share a CU; those of eight waves (115 to 147 KB), where
+//   there are no more workgroups than CUs, and of 32 rows 128 deep (98 KB) have
+//   one to themselves.
 // - A decode step's small kernels are part of the products beside them, as each
 //   alone is a launch of 5-6 us: the RMS norm in front (x enters times the
 //   norm's weights, rounded as the normed row is; its rows' squares are summed
@@ -39,15 +41,6 @@
 #include "common.h"
 #include "lds_dma.h"
 #include "mfma.h"
-
-namespace {
-
-template <int N>
-__device__ __forceinline__ void wait_transfers() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-}  // namespace
 
 // What leaves a product: itself, in bf16 or fp32; silu(gate) * up of [gate; up]
 // stacked; its sum with what y holds; the rotated query, key and value rows,

@@ -29,10 +29,6 @@
 
 namespace {
 
-template <int N>
-__device__ __forceinline__ void wait_transfers() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 // all but the last min(TILES, later) tiles of EACH transfers have landed
 template <int TILES, int EACH>
 __device__ __forceinline__ void wait_all_but(int later) {

@@ -13,6 +13,11 @@ __device__ __forceinline__ void lds_barrier() {
 __device__ __forceinline__ void dma_barrier() {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
+// All but the last N transfers of this wave have landed.
+template <int N>
+__device__ __forceinline__ void wait_transfers() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 // 16 bytes a lane from global memory to LDS at lds (wave-uniform) + 16*lane.
 // As asm: the compiler would let every later LDS read wait for the transfer;
 // here only dma_barrier does. (Wait counts it places for its own loads are

@@ -37,6 +37,24 @@ __device__ __forceinline__ float row16_sum(float v) {
     return v + row16_ror<1>(v);
 }
 
+// maximum / sum over the four lanes that hold one column (l, l^16, l^32, l^48)
+__device__ __forceinline__ float column_max(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(
+        __float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(
+        __float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float column_sum(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(
+        __float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(
+        __float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 // ds_read_b64_tr_b16 twice: a 16-lane group's lanes address 4 rows of 16
 // columns (lane i: row i/4, columns (i%4)*4..+3) and each gets one column
 __device__ __forceinline__ bf16x8 tr_pair(const bf16* lo_rows, const bf16* hi_rows) {
