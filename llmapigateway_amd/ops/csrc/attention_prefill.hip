@@ -5,8 +5,11 @@
 // Produces the prompt phase (TTFT) the reference delegated upstream.
 //
 // - A workgroup has 64 query rows of up to four heads of one kv head: each wave
-//   32 rows of one head, so that a key and value tile staged once serves 256
-//   query columns, and a fragment read from LDS two products.
+//   16 rows of one head, so that a key and value tile staged once serves 256
+//   query columns, and 4 waves a SIMD keep its units busy (with 32 rows a wave,
+//   each fragment from LDS serves two products, but 2 waves a SIMD wait for each
+//   other's exponentials: 4000 tokens after 4032 512 us, 464 so; 1000 tokens 34
+//   and 26).
 // - S^T = K Q^T: a lane owns one query column of a block of 16, its softmax
 //   state is a scalar, and the weights as they stand are the operand of
 //   O^T = V^T P^T (the key order inside a product is free; V fragments come
@@ -19,19 +22,19 @@
 //   a time, scores relative to the largest so far, weights as bf16 (the largest is
 //   1 and loses nothing) for the values and as fp32 for their sum. What a prompt
 //   leaves behind in pages of bytes so depends on the prompt alone. (A maximum
-//   that moves only past 2^8 takes 163 us instead of 185 for 4096 tokens, but
-//   rounds the largest weights, too: over 4000 keys the weights' share of the error
-//   is 1.6e-3 then, 1.25e-3 so.)
+//   that moves only past 2^8 saves a tenth of the time, but rounds the largest
+//   weights, too: over 4000 keys the weights' share of the error is 1.6e-3 then,
+//   1.25e-3 so.)
 // - Blocks of one kv head follow each other at the distance of the XCDs, and
 //   late tiles, which see the most keys, start first.
 //
 // One layer, 32 query and 8 kv heads; before: 64 rows and one head a workgroup,
 // keys and values through registers, weights through LDS:
-//   4096 tokens                   1117 us -> 185 us (743 TFLOP/s)
-//   4000 tokens after 4032        2371    -> 503    (786), e4m3 pages the same
-//   9 x 117-213 tokens after 1984  428    -> 102
-//   32 x 66-128 tokens              46    ->  24
-//   37 tokens                      6.6    -> 6.3
+//   4096 tokens                   1117 us -> 189 us (727 TFLOP/s)
+//   4000 tokens after 4032        2371    -> 464    (852), from e4m3 pages 494
+//   9 x 117-213 tokens after 1984  428    ->  87
+//   32 x 66-128 tokens              46    ->  23
+//   37 tokens                      6.6    -> 6.1
 // Long prompts are bound by the vector ALU beside the matrix cores (an
 // exponential and 6 operations a score, the sums' rescaling).
 
@@ -104,10 +107,10 @@ __device__ __forceinline__ void dequantize16(const uint4& b, float scale, uint4*
 
 }  // namespace
 
-// HG: heads of a workgroup (two waves each); FP8C: pages are e4m3 with a scale
+// HG: heads of a workgroup (four waves each); FP8C: pages are e4m3 with a scale
 // a row.
 template <int HG, bool FP8C>
-__launch_bounds__(HG * 2 * WAVE_SIZE, 2)
+__launch_bounds__(HG * 4 * WAVE_SIZE, 2)
 __global__ void attention_prefill_kernel(
     bf16* __restrict__ out,             // [T, Hq, D]
     const bf16* __restrict__ q,         // [T, Hq, D] (rows strided)
@@ -125,7 +128,7 @@ __global__ void attention_prefill_kernel(
     const int* __restrict__ block_tables,  // [B, max_blocks] or null
     const int* __restrict__ cached_lens,   // [B] or null
     int block_size, int max_blocks) {
-    constexpr int KT = PF_KEYS, NW = 2 * HG, NQ = 2;
+    constexpr int KT = PF_KEYS, NW = 4 * HG;
     constexpr int TILE = KT * PF_ROW;          // bytes of a key or value tile
     constexpr int MOVES = KT / 4;              // 1 KB transfers of one
     constexpr int MINE = (MOVES + NW - 1) / NW;
@@ -141,20 +144,19 @@ __global__ void attention_prefill_kernel(
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, grp = lane >> 4;
-    const int head_in = group * HG + (wave >> 1);  // of the kv head's G
+    const int head_in = group * HG + (wave >> 2); // of the kv head's G
     const bool has_head = head_in < G;
-    const int row0 = tile0 + (wave & 1) * 32;      // of this wave
+    const int row0 = tile0 + (wave & 3) * 16;      // of this wave
     const int Hq = G * Hkv, head = kvh * G + min(head_in, G - 1);
 
     __shared__ __attribute__((aligned(16))) char lds[2][2][TILE];
 
-    bf16x8 qf[NQ][4];
-#pragma unroll
-    for (int n = 0; n < NQ; ++n) {
-        const int r = min(row0 + n * 16 + col, seq_len - 1);
+    bf16x8 qf[4];
+    {
+        const int r = min(row0 + col, seq_len - 1);
         const bf16* p = q + (int64_t)(seq_start + r) * q_stride + (int64_t)head * PF_D + grp * 8;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) qf[n][c] = *reinterpret_cast<const bf16x8*>(p + c * 32);
+        for (int c = 0; c < 4; ++c) qf[c] = *reinterpret_cast<const bf16x8*>(p + c * 32);
     }
 
     const int limit = min(seq_len, tile0 + QTILE);  // keys that the tile sees
@@ -162,11 +164,11 @@ __global__ void attention_prefill_kernel(
     const int n_tiles = n_cached + (limit + KT - 1) / KT;
     const int* table = block_tables != nullptr ? block_tables + (int64_t)seq * max_blocks : nullptr;
 
-    // rows of a tile: transfer i has rows 4i..4i+3, a lane 16 bytes of one; of
-    // bytes, 8 lanes have a row and a wave 8 rows
-    constexpr int PAGE_ROWS = FP8C ? (KT / 8 + NW - 1) / NW : MINE;
+    // rows of a tile: transfer i has rows 4i..4i+3 of keys and of values, a lane 16
+    // bytes of one; of bytes, it has 8 rows of keys, from KT / 8 on of values
+    constexpr int PAGE_ROWS = FP8C ? (KT / 4 + NW - 1) / NW : MINE;
     auto page_row = [&](int j) {  // row in the tile whose page this lane looks up
-        return FP8C ? (wave + j * NW) * 8 + (lane >> 3) : (wave + j * NW) * 4 + grp;
+        return FP8C ? (wave + j * NW) % (KT / 8) * 8 + (lane >> 3) : (wave + j * NW) * 4 + grp;
     };
     int pages[PAGE_ROWS];
     auto look_up = [&](int t) {
@@ -175,26 +177,27 @@ __global__ void attention_prefill_kernel(
             if (t < n_cached)
                 pages[j] = table[min(t * KT + page_row(j), cached - 1) / block_size];
     };
-    uint4 kb[FP8C ? PAGE_ROWS : 1], vb[FP8C ? PAGE_ROWS : 1];
-    float ks[FP8C ? PAGE_ROWS : 1], vs[FP8C ? PAGE_ROWS : 1];
+    uint4 bytes[FP8C ? PAGE_ROWS : 1];
+    float scales[FP8C ? PAGE_ROWS : 1];
 
     auto issue = [&](int t) {
         const uint32_t at = lds_address(&lds[t & 1][0][0]);
         if (t < n_cached) {
 #pragma unroll
             for (int j = 0; j < PAGE_ROWS; ++j) {
+                const int i = wave + j * NW;
+                if (i >= (FP8C ? KT / 4 : MOVES)) continue;
                 const int r = page_row(j);
-                if (r - (FP8C ? lane >> 3 : grp) >= KT) continue;  // uniform
                 const int pos = min(t * KT + r, cached - 1);
                 const int64_t row =
                     ((int64_t)pages[j] * Hkv + kvh) * block_size + pos % block_size;
                 if constexpr (FP8C) {
-                    kb[j] = *reinterpret_cast<const uint4*>(k_cache + row * PF_D + (lane & 7) * 16);
-                    vb[j] = *reinterpret_cast<const uint4*>(v_cache + row * PF_D + (lane & 7) * 16);
-                    ks[j] = k_scale[row];
-                    vs[j] = v_scale[row];
+                    const bool of_keys = i < KT / 8;
+                    bytes[j] = *reinterpret_cast<const uint4*>(
+                        (of_keys ? k_cache : v_cache) + row * PF_D + (lane & 7) * 16);
+                    scales[j] = (of_keys ? k_scale : v_scale)[row];
                 } else {
-                    const uint32_t to = __builtin_amdgcn_readfirstlane(at + (wave + j * NW) * 1024);
+                    const uint32_t to = __builtin_amdgcn_readfirstlane(at + i * 1024);
                     dma16((const bf16*)(k_cache + row * PF_ROW + pf_key_piece(r, col) * 16), to);
                     dma16((const bf16*)(v_cache + row * PF_ROW + pf_value_piece(r, col) * 16), to + TILE);
                 }
@@ -212,47 +215,51 @@ __global__ void attention_prefill_kernel(
             }
         }
     };
-    // tile t lies in LDS as far as this wave brings it
+    // tile t lies in LDS as far as this wave brings it; behind the last key lies
+    // its row again: zero as values, as 0 times an infinity is none of their sum
     auto land = [&](int t) {
+        const int rows = t < n_cached ? cached - t * KT : limit - (t - n_cached) * KT;
+        if (rows < KT && !(FP8C && t < n_cached)) {
+            wait_transfers<0>();
+#pragma unroll
+            for (int j = 0; j < MINE; ++j) {
+                const int i = wave + j * NW, r = i * 4 + grp;
+                if (i < MOVES && r >= rows)
+                    *reinterpret_cast<uint4*>(&lds[t & 1][1][i * 1024 + lane * 16]) =
+                        make_uint4(0, 0, 0, 0);
+            }
+        }
         if (FP8C && t < n_cached) {
-            char* at = &lds[t & 1][0][0];
 #pragma unroll
             for (int j = 0; j < PAGE_ROWS; ++j) {
-                const int r = page_row(j);
-                if (r - (lane >> 3) >= KT) continue;
+                const int i = wave + j * NW, r = page_row(j);
+                if (i >= KT / 4) continue;
+                const bool of_keys = i < KT / 8;
                 uint4 x[2];
-                dequantize16(kb[j], ks[j], x);
+                dequantize16(bytes[j], scales[j], x);
+                if (!of_keys && r >= rows) x[0] = x[1] = make_uint4(0, 0, 0, 0);
+                char* at = lds[t & 1][of_keys ? 0 : 1] + r * PF_ROW;
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
+                for (int h = 0; h < 2; ++h) {
+                    const int piece = (lane & 7) * 2 + h;
                     *reinterpret_cast<uint4*>(
-                        at + r * PF_ROW + pf_key_piece(r, (lane & 7) * 2 + h) * 16) = x[h];
-                dequantize16(vb[j], vs[j], x);
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    *reinterpret_cast<uint4*>(
-                        at + TILE + r * PF_ROW + pf_value_piece(r, (lane & 7) * 2 + h) * 16) = x[h];
+                        at + (of_keys ? pf_key_piece(r, piece) : pf_value_piece(r, piece)) * 16) = x[h];
+                }
             }
         }
     };
 
-    float m[NQ], l[NQ];
-    f32x4 acc[NQ][8];
+    float m = -INFINITY, l = 0.f;
+    f32x4 acc[8];
 #pragma unroll
-    for (int n = 0; n < NQ; ++n) {
-        m[n] = -INFINITY;
-        l[n] = 0.f;
-#pragma unroll
-        for (int d = 0; d < 8; ++d) acc[n][d] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    }
+    for (int d = 0; d < 8; ++d) acc[d] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
     look_up(0);
     issue(0);
     look_up(1);
     // the queries' loads end here, not at their first use inside the loop
 #pragma unroll
-    for (int n = 0; n < NQ; ++n)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(qf[n][c]));
+    for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(qf[c]));
 
     // fragment addresses: row i of a product's first operand is key 8(i/4) + i%4
     // of 32 (+ 4 in the second), piece 4c + grp, so that a lane's scores are those
@@ -274,92 +281,62 @@ __global__ void attention_prefill_kernel(
         }
         const bool fresh = t >= n_cached;
         const int key0 = (fresh ? t - n_cached : t) * KT;
-        // behind the last key lies its row again: 0 times an infinity is none of
-        // the values' sum
-        const int rows = (fresh ? limit : cached) - key0;
-        if (rows < KT) {
-            for (int i = rows * (PF_ROW / 16) + threadIdx.x; i < TILE / 16; i += NW * WAVE_SIZE)
-                reinterpret_cast<uint4*>(lds[t & 1][1])[i] = make_uint4(0, 0, 0, 0);
-            lds_barrier();
-        }
         // rows of this wave behind all keys of the tile: nothing to do
-        if (!has_head || (fresh && key0 > row0 + 31) || row0 >= seq_len) continue;
+        if (!has_head || (fresh && key0 > row0 + 15) || row0 >= seq_len) continue;
         const char* keys = lds[t & 1][0];
         const char* vals = lds[t & 1][1];
 
-        float s[NQ][2][8];  // scores of keys 32c + 8*grp + j
+        float s[2][8];  // scores of keys 32c + 8*grp + j
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                f32x4 p[NQ];
+                f32x4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int n = 0; n < NQ; ++n) p[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                for (int d = 0; d < 4; ++d)
+                    p = mfma16(*reinterpret_cast<const bf16x8*>(
+                                   keys + key_at[d] + (c * 32 + h * 4) * PF_ROW), qf[d], p);
 #pragma unroll
-                for (int d = 0; d < 4; ++d) {
-                    const bf16x8 kf =
-                        *reinterpret_cast<const bf16x8*>(keys + key_at[d] + (c * 32 + h * 4) * PF_ROW);
-#pragma unroll
-                    for (int n = 0; n < NQ; ++n) p[n] = mfma16(kf, qf[n][d], p[n]);
-                }
-#pragma unroll
-                for (int n = 0; n < NQ; ++n)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) s[n][c][h * 4 + r] = p[n][r] * scale;
+                for (int r = 0; r < 4; ++r) s[c][h * 4 + r] = p[r] * scale;
             }
 
         // keys that some row of this wave does not see
-        const int seen = fresh ? row0 + 1 : cached;
-        if (key0 + KT > seen) {
-#pragma unroll
-            for (int n = 0; n < NQ; ++n) {
-                const int most = fresh ? row0 + n * 16 + col : cached - 1;
-#pragma unroll
-                for (int c = 0; c < 2; ++c)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        if (key0 + c * 32 + grp * 8 + j > most) s[n][c][j] = -INFINITY;
-            }
-        }
-
-        float top[NQ];
-#pragma unroll
-        for (int n = 0; n < NQ; ++n) {
-            float x = s[n][0][0];
+        if (key0 + KT > (fresh ? row0 + 1 : cached)) {
+            const int most = fresh ? row0 + col : cached - 1;
 #pragma unroll
             for (int c = 0; c < 2; ++c)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) x = fmaxf(x, s[n][c][j]);
-            top[n] = column_max(x);
+                for (int j = 0; j < 8; ++j)
+                    if (key0 + c * 32 + grp * 8 + j > most) s[c][j] = -INFINITY;
         }
-        float factor[NQ] = {1.f, 1.f};
-        if (__any(top[0] > m[0] || top[1] > m[1])) {
+
+        float top = s[0][0];
 #pragma unroll
-            for (int n = 0; n < NQ; ++n) {
-                const float m_new = fmaxf(m[n], top[n]);
-                factor[n] = __expf(m[n] - (m_new == -INFINITY ? 0.f : m_new));
-                m[n] = m_new;
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-                for (int d = 0; d < 8; ++d)
+            for (int j = 0; j < 8; ++j) top = fmaxf(top, s[c][j]);
+        top = column_max(top);
+        float factor = 1.f;
+        if (__any(top > m)) {
+            const float m_new = fmaxf(m, top);
+            factor = __expf(m - (m_new == -INFINITY ? 0.f : m_new));
+            m = m_new;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[n][d][r] *= factor[n];
-            }
+            for (int d = 0; d < 8; ++d)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[d][r] *= factor;
         }
-        bf16x8 p[NQ][2];
+        bf16x8 p[2];
+        const float base = m == -INFINITY ? 0.f : m;
 #pragma unroll
-        for (int n = 0; n < NQ; ++n) {
-            const float base = m[n] == -INFINITY ? 0.f : m[n];
+        for (int c = 0; c < 2; ++c) {
+            float* e = s[c];
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                float* e = s[n][c];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) e[j] = __expf(e[j] - base);
-                p[n][c] = as_frag(make_uint4(
-                    cvt_pk_bf16(e[0], e[1]), cvt_pk_bf16(e[2], e[3]),
-                    cvt_pk_bf16(e[4], e[5]), cvt_pk_bf16(e[6], e[7])));
-            }
-            l[n] = fmaf(l[n], factor[n], pf_key_sum(s[n]));
+            for (int j = 0; j < 8; ++j) e[j] = __expf(e[j] - base);
+            p[c] = as_frag(make_uint4(cvt_pk_bf16(e[0], e[1]), cvt_pk_bf16(e[2], e[3]),
+                                      cvt_pk_bf16(e[4], e[5]), cvt_pk_bf16(e[6], e[7])));
         }
+        l = fmaf(l, factor, pf_key_sum(s));
 
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
@@ -367,32 +344,26 @@ __global__ void attention_prefill_kernel(
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 const bf16* lo = reinterpret_cast<const bf16*>(vals + at + c * 32 * PF_ROW);
-                const bf16x8 vf = tr_pair(lo, lo + 4 * PF_D);
-#pragma unroll
-                for (int n = 0; n < NQ; ++n) acc[n][d] = mfma16(vf, p[n][c], acc[n][d]);
+                acc[d] = mfma16(tr_pair(lo, lo + 4 * PF_D), p[c], acc[d]);
             }
         }
     }
 
-    if (!has_head) return;
+    const int r = row0 + col;
+    if (!has_head || r >= seq_len || l <= 0.f) return;
+    const float inv = 1.f / l;
+    bf16* o = out + ((int64_t)(seq_start + r) * Hq + head) * PF_D + grp * 4;
 #pragma unroll
-    for (int n = 0; n < NQ; ++n) {
-        const int r = row0 + n * 16 + col;
-        if (r >= seq_len || l[n] <= 0.f) continue;
-        const float inv = 1.f / l[n];
-        bf16* o = out + ((int64_t)(seq_start + r) * Hq + head) * PF_D + grp * 4;
-#pragma unroll
-        for (int d = 0; d < 8; ++d)
-            *reinterpret_cast<uint2*>(o + d * 16) =
-                make_uint2(cvt_pk_bf16(acc[n][d][0] * inv, acc[n][d][1] * inv),
-                           cvt_pk_bf16(acc[n][d][2] * inv, acc[n][d][3] * inv));
-    }
+    for (int d = 0; d < 8; ++d)
+        *reinterpret_cast<uint2*>(o + d * 16) =
+            make_uint2(cvt_pk_bf16(acc[d][0] * inv, acc[d][1] * inv),
+                       cvt_pk_bf16(acc[d][2] * inv, acc[d][3] * inv));
 }
 
 extern "C" hipError_t launch_attention_prefill(
     void* out, const void* q, const void* k, const void* v,
     const int* cu_seqlens, const int* tile_seq, const int* tile_off,
-    int ntiles, int nseq, float scale, int Hq, int Hkv, int D, int64_t q_stride,
+    int ntiles, float scale, int Hq, int Hkv, int D, int64_t q_stride,
     int64_t k_stride, int64_t v_stride, const void* k_cache,
     const void* v_cache, const float* k_scale, const float* v_scale,
     const int* block_tables, const int* cached_lens,
@@ -401,10 +372,10 @@ extern "C" hipError_t launch_attention_prefill(
     if (Hkv <= 0 || Hq % Hkv != 0) return hipErrorInvalidValue;
     if (ntiles <= 0) return hipSuccess;
     const int G = Hq / Hkv;
-#define LAUNCH(HG)                                                       \
+#define LAUNCH(HG)                                                           \
     do {                                                                       \
         const int groups = (G + HG - 1) / HG;                                  \
-        const dim3 grid(Hkv * groups * ntiles), block(HG * 2 * WAVE_SIZE);      \
+        const dim3 grid(Hkv * groups * ntiles), block(HG * 4 * WAVE_SIZE);           \
         if (k_scale != nullptr)                                                \
             attention_prefill_kernel<HG, true><<<grid, block, 0, stream>>>(\
                 (bf16*)out, (const bf16*)q, (const bf16*)k, (const bf16*)v,    \
@@ -420,19 +391,30 @@ extern "C" hipError_t launch_attention_prefill(
                 (const char*)v_cache, k_scale, v_scale, block_tables,          \
                 cached_lens, block_size, max_blocks);                          \
     } while (0)
-    // Heads of a workgroup, by how many workgroups of four heads there would be.
-    // Four (three where that divides the group better) where they fill the 256
-    // CUs; two where CUs would idle, or where sequences are short and latency
-    // counts. 32:8 heads, us with 4 / 2 / 1 heads: 4096 tokens 189 / 199 / 329, 9 x
-    // 117-213 after 1984 106 / 110 / 231, 1000 tokens 44 / 34 / 44, 32 x 66-128 27 /
-    // 24 / 35, 300 tokens 18 / 13 / 16, 37 tokens 7.9 / 6.6 / 7.2. One head a kv
-    // head: the waves without one bring keys (32 heads, 2000 tokens 89 us with two,
-    // 93 with one; 150 tokens after 1000 46 and 66).
-    const int full = ntiles * Hkv * ((G + 3) / 4);
-    const bool short_keys = cached_lens == nullptr && ntiles <= 4 * nseq;
-    if (G <= 2 || full < 160 || short_keys) LAUNCH(2);
-    else if (G == 3 || G == 5 || G == 6) LAUNCH(3);
-    else LAUNCH(4);
+    // Heads of a workgroup: one where that many workgroups run at once or nearly
+    // (512 do), two beyond; with cached rows, where keys are many for all rows, as
+    // many as still give work to half of the 256 CUs. One head a kv head has two,
+    // whose idle waves bring keys. us with 1 / 2 / 3 / 4 heads:
+    //   32:8 heads   300 tokens 10 / 12 / 15 / 17, 1000 26 / 29 / 36 / 42, 1600 46 /
+    //     50 / 60 / 67, 2000 70 / 64 / 83 / 83, 4096 227 / 189 / 275 / 189, 32 x
+    //     66-128 27 / 23 / 33 / 26; after 2000: 3 x 150 73 / 66 / 77 / 85, 6 x 150 132
+    //     / 100 / 153 / 90 (e4m3 170 / 153 / 172 / 99); 4000 after 4032 693 / 503 /
+    //     789 / 464
+    //   24:8 heads   4000 tokens 170 / 164 / 147 / 152
+    //   28:4 heads   1500 tokens 38 / 46 / 55 / 61, 3000 119 / 112 / 118 / 116; 3000
+    //     after 1000 in e4m3 233 / 231 / 203 / 179
+    //   32:32 heads  2000 tokens 68 / 65 / 94 / 85
+    auto groups_of = [&](int heads) { return ntiles * Hkv * ((G + heads - 1) / heads); };
+    if (cached_lens != nullptr && G > 2 && groups_of(4) >= 128) {
+        if (G == 3 || G == 5 || G == 6) LAUNCH(3);
+        else LAUNCH(4);
+    } else if (G > 1 && (cached_lens != nullptr ? groups_of(2) < 128 : groups_of(1) <= 800)) {
+        LAUNCH(1);
+    } else if (G == 3) {
+        LAUNCH(3);
+    } else {
+        LAUNCH(2);
+    }
 #undef LAUNCH
     HIP_CHECK_LAST();
     return hipSuccess;

@@ -13,7 +13,7 @@ hipError_t launch_rope(void*, void*, const int64_t*, const float*, int, int64_t,
 hipError_t launch_kv_cache_write(const void*, const void*, void*, void*, float*, float*, const int64_t*, int, int64_t, int64_t, int, int, int, hipStream_t);
 hipError_t launch_rope_kv(void*, void*, const void*, void*, void*, float*, float*, const int64_t*, const float*, const int64_t*, int, int64_t, int64_t, int64_t, int, int, int, int, hipStream_t);
 hipError_t launch_attention_decode(void*, const void*, const void*, const void*, const float*, const float*, const int*, const int*, float, int, int, int, int, int, int, int64_t, float*, float*, int, hipStream_t);
-hipError_t launch_attention_prefill(void*, const void*, const void*, const void*, const int*, const int*, const int*, int, int, float, int, int, int, int64_t, int64_t, int64_t, const void*, const void*, const float*, const float*, const int*, const int*, int, int, hipStream_t);
+hipError_t launch_attention_prefill(void*, const void*, const void*, const void*, const int*, const int*, const int*, int, float, int, int, int, int64_t, int64_t, int64_t, const void*, const void*, const float*, const float*, const int*, const int*, int, int, hipStream_t);
 hipError_t launch_sample(int64_t*, const float*, const float*, const float*, float*, int*, int, int, hipStream_t);
 hipError_t launch_topk_topp_filter(float*, const float*, const int*, int, int, void*, hipStream_t);
 size_t filter_scratch_bytes(int, int);
@@ -228,7 +228,7 @@ void attention_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
     CHECK_HIP(launch_attention_prefill(
         out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
         cu_seqlens.data_ptr<int>(), tile_seq.data_ptr<int>(),
-        tile_off.data_ptr<int>(), ntiles, (int)cu_seqlens.size(0) - 1, (float)scale, q.size(1), k.size(1),
+        tile_off.data_ptr<int>(), ntiles, (float)scale, q.size(1), k.size(1),
         q.size(2), q.stride(0), k.stride(0), v.stride(0),
         cl ? kc.data_ptr() : nullptr, cl ? vc.data_ptr() : nullptr,
         cl ? scale_ptr(k_scale) : nullptr, cl ? scale_ptr(v_scale) : nullptr,
